@@ -107,30 +107,54 @@ template <int W> UPD_DEV u32 bitlen(const Mag<W>& a)
     return b;
 }
 
+// One limb of a carry or borrow chain (c in and out, 0 or 1).  The clang
+// builtins become one v_addc / v_subb a limb with the carry in VCC; the same
+// chain written with 64-bit sums takes a 64-bit add, two moves and a shift a
+// limb.
+#if defined(__clang__)
+UPD_DEV u32 addc(u32 a, u32 b, u32& c) { return __builtin_addc(a, b, c, &c); }
+UPD_DEV u32 subb(u32 a, u32 b, u32& c) { return __builtin_subc(a, b, c, &c); }
+#else
+UPD_DEV u32 addc(u32 a, u32 b, u32& c)
+{
+    const u64 t = (u64)a + b + c;
+    c = (u32)(t >> 32);
+    return (u32)t;
+}
+UPD_DEV u32 subb(u32 a, u32 b, u32& c)
+{
+    const u64 t = (u64)a - b - c;
+    c = (u32)(t >> 63);
+    return (u32)t;
+}
+#endif
+
+// whether any active lane of the wave has x (the host build has one lane)
+UPD_DEV bool any_lane(bool x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(x) != 0;
+#else
+    return x;
+#endif
+}
+
 // r = a + b, returns carry out
 template <int W> UPD_DEV u32 add_to(Mag<W>& r, const Mag<W>& a, const Mag<W>& b)
 {
-    u64 c = 0;
+    u32 c = 0u;
 #pragma unroll
-    for (int i = 0; i < W; i++) {
-        u64 t = (u64)a.w[i] + b.w[i] + c;
-        r.w[i] = (u32)t;
-        c = t >> 32;
-    }
-    return (u32)c;
+    for (int i = 0; i < W; i++) r.w[i] = addc(a.w[i], b.w[i], c);
+    return c;
 }
 
 // r = a - b, returns borrow out (1 when a < b)
 template <int W> UPD_DEV u32 sub_to(Mag<W>& r, const Mag<W>& a, const Mag<W>& b)
 {
-    u64 br = 0;
+    u32 br = 0u;
 #pragma unroll
-    for (int i = 0; i < W; i++) {
-        u64 t = (u64)a.w[i] - b.w[i] - br;
-        r.w[i] = (u32)t;
-        br = (t >> 63) & 1u;
-    }
-    return (u32)br;
+    for (int i = 0; i < W; i++) r.w[i] = subb(a.w[i], b.w[i], br);
+    return br;
 }
 
 // -1, 0, 1
@@ -198,7 +222,8 @@ template <int W> UPD_DEV Mag<W> shl_var(const Mag<W>& a, u32 k)
     Mag<W> t = a;
 #pragma unroll
     for (int st = 1; st < W; st <<= 1) {
-        bool on = (ws & (u32)st) != 0;
+        const bool on = (ws & (u32)st) != 0;
+        if (!any_lane(on)) continue;  // a stage no lane of the wave needs
         Mag<W> u;
 #pragma unroll
         for (int i = 0; i < W; i++) u.w[i] = (i >= st) ? t.w[i - st] : 0u;
@@ -221,7 +246,8 @@ template <int W> UPD_DEV Mag<W> shr_var(const Mag<W>& a, u32 k)
     Mag<W> t = a;
 #pragma unroll
     for (int st = 1; st < W; st <<= 1) {
-        bool on = (ws & (u32)st) != 0;
+        const bool on = (ws & (u32)st) != 0;
+        if (!any_lane(on)) continue;  // a stage no lane of the wave needs
         Mag<W> u;
 #pragma unroll
         for (int i = 0; i < W; i++) u.w[i] = (i + st < W) ? t.w[i + st] : 0u;
@@ -268,12 +294,50 @@ UPD_DEV u32 div_2by1(u32 u1, u32 u0, u32 d, u32 v, u32& r)
     return q1;
 }
 
+// Reciprocal of a normalized two-word divisor (d1, d0), top bit of d1 set:
+// floor((2^96 - 1) / (d1 2^32 + d0)) - 2^32 (Moller & Granlund 2011,
+// Algorithm 6, from the one-word reciprocal).
+UPD_DEV u32 recip_2word(u32 d1, u32 d0)
+{
+    u32 v = recip_word(d1);
+    u32 p = d1 * v + d0;
+    if (p < d0) {
+        v -= 1u;
+        if (p >= d1) {
+            v -= 1u;
+            p -= d1;
+        }
+        p -= d1;
+    }
+    const u64 t = (u64)v * d0;
+    p += (u32)(t >> 32);
+    if (p < (u32)(t >> 32)) {
+        v -= 1u;
+        if ((((u64)p << 32) | (u32)t) >= (((u64)d1 << 32) | d0)) v -= 1u;
+    }
+    return v;
+}
+
 // Q = floor(X / B), R = X mod B, for B != 0.  Knuth, TAOCP vol. 2, 4.3.1,
 // Algorithm D, with the divisor normalized to fill all NB limbs (so the
-// quotient loop has a static trip count of NX+1 digits) and the digit
-// estimate from div_2by1 refined by the second divisor limb.
-// One quotient digit of Knuth's Algorithm D (TAOCP 4.3.1): digit J of the
-// quotient from the window un[J .. J+NB] and the normalized divisor vn.
+// quotient loop has a static trip count of NX+1 digits).
+//
+// One quotient digit: digit J of the quotient from the window
+// un[J .. J+NB] and the normalized divisor vn (top words d1, d0; v their
+// reciprocal: of d1 alone when NB = 1, else of (d1, d0)).  The digit is the
+// exact quotient of the window's three top words by (d1, d0) (Moller &
+// Granlund 2011, Algorithm 4), so it is at most one too large for the whole
+// window (TAOCP 4.3.1, exercise 20), with probability about 2^-32; the
+// division also leaves the top two words of the new window, and only the
+// other NB - 2 limbs are multiplied and subtracted.
+//
+// Integer VALU bounds it.  A limb of the subtraction is three instructions:
+// a multiply-add that carries the high word along (v_mad_u64_u32), the move
+// that zero-extends that word, and v_subb.  Written with 64-bit differences it had been
+// ten, and the digit estimate a two-word quotient with two corrections in
+// branches: x * x % N * x % N with 71-digit N, 3 M rows, 189 -> 136 us; the
+// P = 300 sweep expression, 1 M rows, 792 -> 688 us; P = 150, 2 M rows, 273 ->
+// 247 us.
 template <int J, int NB, int NU>
 UPD_DEV u32 divmod_digit(Mag<NU>& un, const Mag<NB>& vn, u32 d1, u32 d0, u32 v)
 {
@@ -282,55 +346,58 @@ UPD_DEV u32 divmod_digit(Mag<NU>& un, const Mag<NB>& vn, u32 d1, u32 d0, u32 v)
     // changes (the top digits of a dividend narrower than its static width;
     // a wave-uniform branch in practice)
     if (u2 == 0u && u1 < d1) return 0u;
-    u32 qhat;
-    u64 rhat;
-    if (u2 >= d1) {
-        qhat = 0xffffffffu;
-        rhat = (u64)u1 + d1;
+    if constexpr (NB == 1) {
+        u32 r;
+        const u32 q = div_2by1(u2, u1, d1, v, r);
+        un.w[J] = r;
+        un.w[J + 1] = 0u;
+        return q;
     } else {
-        u32 r32;
-        qhat = div_2by1(u2, u1, d1, v, r32);
-        rhat = r32;
-    }
-    if constexpr (NB >= 2) {
         const u32 u0 = un.w[J + NB - 2];
-#pragma unroll
-        for (int it = 0; it < 2; it++) {
-            bool fix = (rhat < (1ull << 32)) && ((u64)qhat * d0 > ((rhat << 32) | u0));
-            qhat -= fix ? 1u : 0u;
-            rhat += fix ? d1 : 0u;
+        const u64 D = ((u64)d1 << 32) | d0;
+        const u64 qe = (u64)v * u2 + (((u64)u2 << 32) | u1);
+        u32 q = (u32)(qe >> 32);
+        u64 r = ((((u64)u1 << 32) | u0) - D) - (u64)q * d0 - ((u64)(q * d1) << 32);
+        q += 1u;
+        if ((u32)(r >> 32) >= (u32)qe) {
+            q -= 1u;
+            r += D;
         }
-    }
-    // un[J .. J+NB] -= qhat * vn.  A zero digit changes nothing: the top
-    // digits of a dividend shorter than its static width are all zero, and
-    // skipping them (a wave-uniform branch when every lane's digit is zero)
-    // removes most of the work of a wide division
-    if (qhat != 0u) {
-        u64 kk = 0;
-        i64 t;
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            u64 p = (u64)qhat * vn.w[i];
-            t = (i64)un.w[i + J] - (i64)kk - (i64)(p & 0xffffffffull);
-            un.w[i + J] = (u32)t;
-            kk = (p >> 32) - (u64)(t >> 32);
+        if (r >= D) {
+            q += 1u;
+            r -= D;
         }
-        t = (i64)un.w[J + NB] - (i64)kk;
-        un.w[J + NB] = (u32)t;
-        // rare add-back when the estimate was one too large
-        if (t < 0) {
-            qhat -= 1u;
-            u64 c = 0;
-#pragma unroll
-            for (int i = 0; i < NB; i++) {
-                u64 s = (u64)un.w[i + J] + vn.w[i] + c;
-                un.w[i + J] = (u32)s;
-                c = s >> 32;
+        if constexpr (NB > 2) {
+            // top words equal: the quotient word saturates, and the top of
+            // the new window is (d1, d0) + u0, a third word when it carries
+            u32 r2 = 0u;
+            if (u2 == d1 && u1 == d0) {
+                q = 0xffffffffu;
+                r = D + u0;
+                r2 = r < D ? 1u : 0u;
             }
-            un.w[J + NB] += (u32)c;
+            u32 cy = 0u, br = 0u;
+#pragma unroll
+            for (int i = 0; i < NB - 2; i++) {
+                const u64 p = (u64)q * vn.w[i] + cy;
+                cy = (u32)(p >> 32);
+                un.w[i + J] = subb(un.w[i + J], (u32)p, br);
+            }
+            un.w[J + NB - 2] = subb((u32)r, cy, br);
+            un.w[J + NB - 1] = subb((u32)(r >> 32), 0u, br);
+            // rare add-back when the digit was one too large
+            if (br > r2) {
+                q -= 1u;
+                u32 c = 0u;
+#pragma unroll
+                for (int i = 0; i < NB; i++) un.w[i + J] = addc(un.w[i + J], vn.w[i], c);
+            }
+        } else {
+            un.w[J] = (u32)r;
+            un.w[J + 1] = (u32)(r >> 32);
         }
+        return q;
     }
-    return qhat;
 }
 
 // digits J, J-1, ..., 0, each its own instantiation: every limb index is a
@@ -352,7 +419,7 @@ template <int NX, int NB> UPD_DEV void divmod(const Mag<NX>& X, const Mag<NB>& B
     Mag<NU> un = shl_var<NU>(resize<NU>(X), k);
     const u32 d1 = vn.w[NB - 1];
     const u32 d0 = (NB >= 2) ? vn.w[NB - 2] : 0u;
-    const u32 v = recip_word(d1);
+    const u32 v = NB >= 2 ? recip_2word(d1, d0) : recip_word(d1);
     divmod_digits<NX, NB, NU, NX + 1>(un, vn, d1, d0, v, Q);
     R = shr_var<NB>(resize<NB>(un), k);
 }
