@@ -166,50 +166,55 @@ template <int W> UPD_DEV int cmp(const Mag<W>& a, const Mag<W>& b)
     return c;
 }
 
-// low WO limbs of a * b (schoolbook, 32x32->64 multiply-accumulate)
+// a >= b
+template <int W> UPD_DEV bool ge(const Mag<W>& a, const Mag<W>& b)
+{
+    u32 br = 0u;
+#pragma unroll
+    for (int i = 0; i < W; i++) (void)subb(a.w[i], b.w[i], br);
+    return br == 0u;
+}
+
+// Row I of a schoolbook product: r += x * b * 2^(32 I), and the rows after
+// it.  A limb product is one multiply-add that carries the high word along,
+// the move that zero-extends that word, and one v_addc.  Every row is its
+// own instantiation: a row loop that the compiler leaves rolled (it did for
+// 32 x 32 limbs) indexes the operands at run time and moves them to memory
+// (LDS, or 388 bytes of scratch a lane).
+template <int I, int WO, int WA, int WB, class B> UPD_DEV void mul_rows(Mag<WO>& r, const Mag<WA>& a, const B& b)
+{
+    if constexpr (I < WA && I < WO) {
+        u32 hi = 0u, c = 0u;
+#pragma unroll
+        for (int j = 0; j < WB; j++) {
+            if (I + j < WO) {
+                const u64 t = (u64)a.w[I] * b.w[j] + hi;
+                hi = (u32)(t >> 32);
+                r.w[I + j] = I == 0 ? (u32)t : addc(r.w[I + j], (u32)t, c);
+            }
+        }
+        if (I + WB < WO) r.w[I + WB] = hi + c;
+        mul_rows<I + 1, WO, WA, WB, B>(r, a, b);
+    }
+}
+
+// low WO limbs of a * b
 template <int WO, int WA, int WB> UPD_DEV Mag<WO> mul_lo(const Mag<WA>& a, const Mag<WB>& b)
 {
     Mag<WO> r = mzero<WO>();
-#pragma unroll
-    for (int i = 0; i < WA; i++) {
-        if (i >= WO) break;
-        u64 c = 0;
-#pragma unroll
-        for (int j = 0; j < WB; j++) {
-            if (i + j < WO) {
-                u64 t = (u64)a.w[i] * b.w[j] + r.w[i + j] + c;
-                r.w[i + j] = (u32)t;
-                c = t >> 32;
-            }
-        }
-        if (i + WB < WO) r.w[i + WB] = (u32)c;
-    }
+    mul_rows<0, WO, WA, WB, Mag<WB>>(r, a, b);
     return r;
 }
 
-// low WO limbs of a * 10^N (constant row, zero limbs of 10^N skipped)
+// low WO limbs of a * 10^N (constant row)
 template <int WO, int WA, int N> UPD_DEV Mag<WO> mul_p10(const Mag<WA>& a)
 {
     if constexpr (N == 0) {
         return resize<WO>(a);
     } else {
         constexpr BigConst p = P10<N>::c;
-        constexpr int WP = P10<N>::W;
         Mag<WO> r = mzero<WO>();
-#pragma unroll
-        for (int i = 0; i < WA; i++) {
-            if (i >= WO) break;
-            u64 c = 0;
-#pragma unroll
-            for (int j = 0; j < WP; j++) {
-                if (i + j < WO) {
-                    u64 t = (u64)a.w[i] * p.w[j] + r.w[i + j] + c;
-                    r.w[i + j] = (u32)t;
-                    c = t >> 32;
-                }
-            }
-            if (i + WP < WO) r.w[i + WP] = (u32)c;
-        }
+        mul_rows<0, WO, WA, P10<N>::W, BigConst>(r, a, p);
         return r;
     }
 }
@@ -333,11 +338,9 @@ UPD_DEV u32 recip_2word(u32 d1, u32 d0)
 //
 // Integer VALU bounds it.  A limb of the subtraction is three instructions:
 // a multiply-add that carries the high word along (v_mad_u64_u32), the move
-// that zero-extends that word, and v_subb.  Written with 64-bit differences it had been
-// ten, and the digit estimate a two-word quotient with two corrections in
-// branches: x * x % N * x % N with 71-digit N, 3 M rows, 189 -> 136 us; the
-// P = 300 sweep expression, 1 M rows, 792 -> 688 us; P = 150, 2 M rows, 273 ->
-// 247 us.
+// that zero-extends that word, and v_subb.  Written with 64-bit differences
+// it had been ten, and the digit estimate a two-word quotient with two
+// corrections in branches.
 template <int J, int NB, int NU>
 UPD_DEV u32 divmod_digit(Mag<NU>& un, const Mag<NB>& vn, u32 d1, u32 d0, u32 v)
 {
@@ -411,17 +414,28 @@ UPD_DEV void divmod_digits(Mag<NU>& un, const Mag<NB>& vn, u32 d1, u32 d0, u32 v
     if constexpr (J > 0) divmod_digits<J - 1, NB, NU, NQ>(un, vn, d1, d0, v, Q);
 }
 
-template <int NX, int NB> UPD_DEV void divmod(const Mag<NX>& X, const Mag<NB>& B, Mag<NX + 1>& Q, Mag<NB>& R)
+// the division up to the shift back: Rn = R 2^k and vn = B 2^k, k the shift
+// that fills vn's top bit
+template <int NX, int NB>
+UPD_DEV void divmod_norm(const Mag<NX>& X, const Mag<NB>& B, Mag<NX + 1>& Q, Mag<NB>& Rn, Mag<NB>& vn, u32& k)
 {
     constexpr int NU = NX + NB + 1;
-    const u32 k = 32u * NB - bitlen(B);
-    const Mag<NB> vn = shl_var<NB>(B, k);
+    k = 32u * NB - bitlen(B);
+    vn = shl_var<NB>(B, k);
     Mag<NU> un = shl_var<NU>(resize<NU>(X), k);
     const u32 d1 = vn.w[NB - 1];
     const u32 d0 = (NB >= 2) ? vn.w[NB - 2] : 0u;
     const u32 v = NB >= 2 ? recip_2word(d1, d0) : recip_word(d1);
     divmod_digits<NX, NB, NU, NX + 1>(un, vn, d1, d0, v, Q);
-    R = shr_var<NB>(resize<NB>(un), k);
+    Rn = resize<NB>(un);
+}
+
+template <int NX, int NB> UPD_DEV void divmod(const Mag<NX>& X, const Mag<NB>& B, Mag<NX + 1>& Q, Mag<NB>& R)
+{
+    u32 k;
+    Mag<NB> Rn, vn;
+    divmod_norm<NX, NB>(X, B, Q, Rn, vn, k);
+    R = shr_var<NB>(Rn, k);
 }
 
 // ---------------------------------------------------------------- signed operations
@@ -789,61 +803,61 @@ template <int W> UPD_DEV Dec<W> ddiv_rt(const Dec<W>& a, const Dec<W>& b, u32 S,
 {
     const bool azero = is_zero(a.m);
     const bool bzero = is_zero(b.m);
+    Mag<W> X = mul_p10_rt<W>(a.m, S);
     Mag<W> bs = b.m;
-    if (bzero) bs.w[0] = 1u;
-    const Mag<W> X = mul_p10_rt<W>(a.m, S);
-    Mag<W + 1> Q;
-    Mag<W> R;
-    divmod<W, W>(X, bs, Q, R);
-    Mag<W> T;
-    sub_to<W>(T, bs, R);
-    u32 rnd = cmp<W>(R, T) >= 0 ? 1u : 0u;
-    if (faith) {
-        const u32 bla = bitlen(a.m), blb = bitlen(bs);
-        const bool path_i = (bla + (u32)est_shift_bits((int)S) - 1u <= 64u) && blb <= 64u;
-        bool top0 = true;
+    // x / 0 keeps |x|: the unscaled dividend divided by 1.  Neither operand
+    // is kept through the division (the rounding below works on the
+    // normalized remainder): at P = 300 that and the operand loads of 16
+    // bytes take the sweep expression, 1 M rows, from 688 to 454 us, with the
+    // unrolled product's rows (71-digit x*x%N*x%N, 3 M rows: 136 to 120)
+    if (any_lane(bzero)) {
+        bs.w[0] |= bzero ? 1u : 0u;
 #pragma unroll
-        for (int i = 1; i < W; i++) top0 = top0 && bs.w[i] == 0u;
-        const bool path_ii = !path_i && top0;
-        const u32 blx = bitlen(X);
-        const bool path_iii_one = !path_i && !path_ii && blx < blb && blb - blx <= 64u;
-        if (path_ii) rnd = ((u32)(R.w[0] * 2u) >= bs.w[0]) ? 1u : 0u;
+        for (int i = 0; i < W; i++) X.w[i] = bzero ? (i < W ? a.m.w[i] : 0u) : X.w[i];
+    }
+    bool path_i = false, path_ii = false, path_iii_one = false;
+    Mag<2> a2 = resize<2>(a.m), b2 = resize<2>(bs);
+    if (faith) {
+        const u32 bla = bitlen(a.m), blb = bitlen(bs), blx = bitlen(X);
+        path_i = !bzero && bla + (u32)est_shift_bits((int)S) - 1u <= 64u && blb <= 64u;
+        path_ii = !path_i && blb <= 32u;
+        path_iii_one = !path_i && !path_ii && blx < blb && blb - blx <= 64u;
+    }
+    Mag<W + 1> Q;
+    Mag<W> Rn, vn, T;
+    u32 k;
+    divmod_norm<W, W>(X, bs, Q, Rn, vn, k);
+    // 2 R >= b, tested on the normalized remainder and divisor
+    sub_to<W>(T, vn, Rn);
+    u32 rnd = ge(Rn, T) ? 1u : 0u;
+    if (faith) {
+        // one-word divisor: the remainder is the top word of Rn
+        if (path_ii) rnd = (u32)((Rn.w[W - 1] >> (k & 31u)) * 2u) >= b2.w[0] ? 1u : 0u;
         if (path_iii_one) {
             Q = mzero<W + 1>();
             Q.w[0] = 1u;
             rnd = 0u;
         }
         if (path_i) {
-            Mag<2> dvs = mul_p10_rt<2>(resize<2>(a.m), S);
-            Mag<2> dvt = resize<2>(bs);
+            // uint64 emulation of DivByInt64 (decimal.cu:2431-2446)
+            const Mag<2> dvs = mul_p10_rt<2>(a2, S);
             Mag<3> q3;
             Mag<2> r2;
-            divmod<2, 2>(dvs, dvt, q3, r2);
+            divmod<2, 2>(dvs, b2, q3, r2);
             Mag<2> r2d;
             r2d.w[0] = r2.w[0] << 1;
             r2d.w[1] = (r2.w[1] << 1) | (r2.w[0] >> 31);
-            rnd = cmp<2>(r2d, dvt) >= 0 ? 1u : 0u;
+            rnd = ge(r2d, b2) ? 1u : 0u;
             Q = resize<W + 1>(resize<2>(q3));
         }
     }
-    u64 c = rnd;
+    // Q += rnd
+    u32 c = rnd;
 #pragma unroll
-    for (int i = 0; i < W + 1; i++) {
-        u64 s = (u64)Q.w[i] + c;
-        Q.w[i] = (u32)s;
-        c = s >> 32;
-    }
+    for (int i = 0; i < W + 1; i++) Q.w[i] = addc(Q.w[i], 0u, c);
     Dec<W> r;
-    if (azero) {
-        r.m = mzero<W>();
-        r.neg = 0u;
-    } else if (bzero) {
-        r.m = a.m;
-        r.neg = a.neg ^ b.neg;
-    } else {
-        r.m = resize<W>(Q);
-        r.neg = a.neg ^ b.neg;
-    }
+    r.m = resize<W>(Q);  // zero for 0 / x, also for 0 / 0
+    r.neg = azero ? 0u : a.neg ^ b.neg;
     return r;
 }
 
@@ -993,25 +1007,36 @@ UPD_DEV Dec<WO> ddiv(const Dec<WA>& a, const Dec<WB>& b, u32* err = nullptr)
     constexpr int WX = WA + P10<S>::W;
     const bool azero = is_zero(a.m);
     const bool bzero = is_zero(b.m);
+    Mag<WX> X = mul_p10<WX, WA, S>(a.m);
     Mag<WB> bs = b.m;
-    if (bzero) bs.w[0] = 1u;
-    const Mag<WX> X = mul_p10<WX, WA, S>(a.m);
-    Mag<WX + 1> Q;
-    Mag<WB> R;
-    divmod<WX, WB>(X, bs, Q, R);
-    Mag<WB> T;
-    sub_to<WB>(T, bs, R);
-    u32 rnd = cmp<WB>(R, T) >= 0 ? 1u : 0u;
-    if constexpr (FAITH) {
-        const u32 bla = bitlen(a.m), blb = bitlen(bs);
-        const bool path_i = (bla + (u32)est_shift_bits(S) - 1u <= 64u) && blb <= 64u;
-        bool top0 = true;
+    // x / 0 keeps |x|: the unscaled dividend divided by 1.  Neither operand
+    // is kept through the division (the rounding below works on the
+    // normalized remainder): at P = 300 that and the operand loads of 16
+    // bytes take the sweep expression, 1 M rows, from 688 to 454 us, with the
+    // unrolled product's rows (71-digit x*x%N*x%N, 3 M rows: 136 to 120)
+    if (any_lane(bzero)) {
+        bs.w[0] |= bzero ? 1u : 0u;
 #pragma unroll
-        for (int i = 1; i < WB; i++) top0 = top0 && bs.w[i] == 0u;
-        const bool path_ii = !path_i && top0;
-        const u32 blx = bitlen(X);
-        const bool path_iii_one = !path_i && !path_ii && blx < blb && blb - blx <= 64u;
-        if (path_ii) rnd = ((u32)(R.w[0] * 2u) >= bs.w[0]) ? 1u : 0u;
+        for (int i = 0; i < WX; i++) X.w[i] = bzero ? (i < WA ? a.m.w[i] : 0u) : X.w[i];
+    }
+    bool path_i = false, path_ii = false, path_iii_one = false;
+    Mag<2> a2 = resize<2>(a.m), b2 = resize<2>(bs);
+    if constexpr (FAITH) {
+        const u32 bla = bitlen(a.m), blb = bitlen(bs), blx = bitlen(X);
+        path_i = !bzero && bla + (u32)est_shift_bits(S) - 1u <= 64u && blb <= 64u;
+        path_ii = !path_i && blb <= 32u;
+        path_iii_one = !path_i && !path_ii && blx < blb && blb - blx <= 64u;
+    }
+    Mag<WX + 1> Q;
+    Mag<WB> Rn, vn, T;
+    u32 k;
+    divmod_norm<WX, WB>(X, bs, Q, Rn, vn, k);
+    // 2 R >= b, tested on the normalized remainder and divisor
+    sub_to<WB>(T, vn, Rn);
+    u32 rnd = ge(Rn, T) ? 1u : 0u;
+    if constexpr (FAITH) {
+        // one-word divisor: the remainder is the top word of Rn
+        if (path_ii) rnd = (u32)((Rn.w[WB - 1] >> (k & 31u)) * 2u) >= b2.w[0] ? 1u : 0u;
         if (path_iii_one) {
             Q = mzero<WX + 1>();
             Q.w[0] = 1u;
@@ -1019,39 +1044,25 @@ UPD_DEV Dec<WO> ddiv(const Dec<WA>& a, const Dec<WB>& b, u32* err = nullptr)
         }
         if (path_i) {
             // uint64 emulation of DivByInt64 (decimal.cu:2431-2446)
-            Mag<2> a2 = resize<2>(a.m);
-            Mag<2> dvs = mul_p10<2, 2, S>(a2);
-            Mag<2> dvt = resize<2>(bs);
+            const Mag<2> dvs = mul_p10<2, 2, S>(a2);
             Mag<3> q3;
             Mag<2> r2;
-            divmod<2, 2>(dvs, dvt, q3, r2);
+            divmod<2, 2>(dvs, b2, q3, r2);
             Mag<2> r2d;
             r2d.w[0] = r2.w[0] << 1;
             r2d.w[1] = (r2.w[1] << 1) | (r2.w[0] >> 31);
-            rnd = cmp<2>(r2d, dvt) >= 0 ? 1u : 0u;
+            rnd = ge(r2d, b2) ? 1u : 0u;
             Q = resize<WX + 1>(resize<2>(q3));
         }
     }
     // Q += rnd
-    u64 c = rnd;
+    u32 c = rnd;
 #pragma unroll
-    for (int i = 0; i < WX + 1; i++) {
-        u64 s = (u64)Q.w[i] + c;
-        Q.w[i] = (u32)s;
-        c = s >> 32;
-    }
+    for (int i = 0; i < WX + 1; i++) Q.w[i] = addc(Q.w[i], 0u, c);
+    if (bzero && !azero && err) *err = 2u;
     Dec<WO> r;
-    if (azero) {
-        r.m = mzero<WO>();
-        r.neg = 0u;
-    } else if (bzero) {
-        r.m = resize<WO>(a.m);
-        r.neg = a.neg ^ b.neg;
-        if (err) *err = 2u;
-    } else {
-        r.m = resize<WO>(Q);
-        r.neg = a.neg ^ b.neg;
-    }
+    r.m = resize<WO>(Q);  // zero for 0 / x, also for 0 / 0
+    r.neg = azero ? 0u : a.neg ^ b.neg;
     return r;
 }
 
@@ -1108,45 +1119,66 @@ template <int WO, int WA, int WB, int FAITH> UPD_DEV Dec<WO> dmod(const Dec<WA>&
 
 // ---------------------------------------------------------------- compact codec
 
+typedef unsigned int u32x4u __attribute__((vector_size(16), aligned(4)));
+typedef unsigned int u32x2u __attribute__((vector_size(8), aligned(4)));
+
 // Decode one compact DECIMAL row (decimal.cu:168-176): B little-endian bytes
 // at row*B, sign in bit 7 of the last byte.  Loads are the aligned dwords
 // covering the row; the last rows of a column, whose covering dwords would
 // run past the column, take a byte path.
-// Decode the B-byte compact value at byte offset `off` of a 4-byte aligned
-// buffer of `colbytes` bytes (load_compact below: off = row * B).
-template <int B> UPD_DEV Dec<(B + 3) / 4> load_compact_off(const u8* __restrict__ col, usize off, usize colbytes)
+// N dwords from a 4-byte aligned address, by 16-byte loads
+template <int N> UPD_DEV void load_dwords(const u32* p, u32* dw)
 {
-    constexpr int ND = (B + 6) / 4;
+#pragma unroll
+    for (int i = 0; i + 4 <= N; i += 4) {
+        const u32x4u v = __builtin_nontemporal_load(reinterpret_cast<const u32x4u*>(p + i));
+        dw[i] = v[0];
+        dw[i + 1] = v[1];
+        dw[i + 2] = v[2];
+        dw[i + 3] = v[3];
+    }
+    if constexpr ((N & 3) >= 2) {
+        const u32x2u v = __builtin_nontemporal_load(reinterpret_cast<const u32x2u*>(p + (N & ~3)));
+        dw[N & ~3] = v[0];
+        dw[(N & ~3) + 1] = v[1];
+    }
+    if constexpr ((N & 1) != 0) dw[N - 1] = __builtin_nontemporal_load(p + (N - 1));
+}
+
+// Decode the B-byte compact value at byte offset `off` of a 4-byte aligned
+// buffer of `colbytes` bytes (load_compact below: off = row * B; ALIGNED:
+// off is a multiple of 4).  The loads are 16 bytes wide: lanes are B bytes
+// apart, so every load instruction touches up to 64 cache lines, and the
+// number of instructions is what a wide row costs.
+template <int B, bool ALIGNED = false>
+UPD_DEV Dec<(B + 3) / 4> load_compact_off(const u8* __restrict__ col, usize off, usize colbytes)
+{
     constexpr int NW = (B + 3) / 4;
+    constexpr int ND = ALIGNED ? NW : (B + 6) / 4;
     const usize d0 = off >> 2;
-    const u32 sh = (u32)(off & 3u);
+    const u32 sh = ALIGNED ? 0u : (u32)(off & 3u);
+    const u32* p = reinterpret_cast<const u32*>(col) + d0;
     u32 dw[ND + 1];
     if ((d0 + ND) * 4u <= colbytes) {
-        const u32* p = reinterpret_cast<const u32*>(col) + d0;
+        load_dwords<NW>(p, dw);
         // the last dword is read only when the row reaches into it: a row
         // that ends on a dword boundary would otherwise touch the next
         // row's dword (and, at the end of a block's range, a cache line
         // another block on another XCD fetches again)
-        const u32 nd = (sh + (u32)B + 3u) >> 2;
-#pragma unroll
-        for (int i = 0; i < ND; i++) dw[i] = (i < NW || (u32)i < nd) ? __builtin_nontemporal_load(p + i) : 0u;
+        if constexpr (ND > NW) dw[NW] = NW < (int)((sh + (u32)B + 3u) >> 2) ? __builtin_nontemporal_load(p + NW) : 0u;
     } else {
+        // the column's last rows: whole dwords inside it, then the bytes of
+        // its partial last dword
+        const usize whole = colbytes >> 2;
+        u32 last = 0;
+        for (usize o = whole * 4u; o < colbytes; o++) last |= (u32)col[o] << (8u * (u32)(o & 3u));
 #pragma unroll
-        for (int i = 0; i < ND; i++) {
-            u32 x = 0;
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                usize o = (d0 + i) * 4u + b;
-                u32 byte = (o < colbytes) ? (u32)col[o] : 0u;
-                x |= byte << (8 * b);
-            }
-            dw[i] = x;
-        }
+        for (int i = 0; i < ND; i++) dw[i] = d0 + (usize)i < whole ? p[i] : (d0 + (usize)i == whole ? last : 0u);
     }
     dw[ND] = 0u;
     Dec<NW> r;
 #pragma unroll
-    for (int i = 0; i < NW; i++) r.m.w[i] = __builtin_amdgcn_alignbyte(dw[i + 1], dw[i], sh);
+    for (int i = 0; i < NW; i++) r.m.w[i] = ALIGNED ? dw[i] : __builtin_amdgcn_alignbyte(dw[i + 1], dw[i], sh);
     if constexpr ((B % 4) != 0) r.m.w[NW - 1] &= (1u << (8 * (B % 4))) - 1u;
     constexpr int SB = 8 * ((B - 1) % 4) + 7;
     r.neg = (r.m.w[NW - 1] >> SB) & 1u;
@@ -1156,7 +1188,7 @@ template <int B> UPD_DEV Dec<(B + 3) / 4> load_compact_off(const u8* __restrict_
 
 template <int B> UPD_DEV Dec<(B + 3) / 4> load_compact(const u8* __restrict__ col, usize row, usize colbytes)
 {
-    return load_compact_off<B>(col, row * (usize)B, colbytes);
+    return load_compact_off<B, B % 4 == 0>(col, row * (usize)B, colbytes);
 }
 
 // ---- wave-staged loads
@@ -1225,8 +1257,6 @@ template <int B> UPD_DEV Dec<(B + 3) / 4> load_staged(const u32* lds, u32 lane)
 // decodes its four rows from registers at byte offsets fixed at compile
 // time once the caller's loop over the four rows is unrolled.
 
-typedef unsigned int u32x4u __attribute__((vector_size(16), aligned(4)));
-typedef unsigned int u32x2u __attribute__((vector_size(8), aligned(4)));
 
 template <int B> struct Quad {
     u32 w[B];

@@ -1756,13 +1756,20 @@ static int plan_peak_limbs(const Plan& p)
     return peak;
 }
 
-// A calc kernel whose plan keeps 48 or more limbs live runs one wave per
-// SIMD with the whole register file (512 VGPRs): at the default occupancy
-// target the compiler keeps those limb arrays partly in scratch (P = 300
-// sweep: 388 B per lane, 16.3 ms per 10 M rows; one wave per SIMD: no
-// scratch, 8.6 ms).  Narrower plans keep the default (P = 150: 1.6 ms, one
-// wave per SIMD would be 2.5 ms).
-static bool calc_one_wave(const Plan& p) { return plan_peak_limbs(p) >= 48; }
+// Waves per SIMD of a calc kernel, by the limbs its plan keeps live (0: the
+// compiler's choice).  64 or more take the whole register file (512 VGPRs):
+// with two waves the limb arrays spill (sweep expression, P = 300, 76 limbs,
+// 1 M rows: 507 against 776 us; P = 260, 65 limbs: 390 against 440).  48 to
+// 63 fit the half that two waves leave each, and the second wave hides the
+// first one's column loads (P = 220, 55 limbs, 1 M rows: 219 against 287 us
+// with one; P = 190, 48 limbs, 1.5 M rows: 254 against 348).  Below that the
+// compiler's choice is as fast or faster (P = 150, 2 M rows: 242 against
+// 252 us; P = 110: 133 against 159).
+static int calc_waves(const Plan& p)
+{
+    const int peak = plan_peak_limbs(p);
+    return peak >= 64 ? 1 : peak >= 48 ? 2 : 0;
+}
 
 std::string gen_calc_kernel(const Plan& p, const std::vector<ColumnType>& cols, const std::string& name, const GenOptions& o)
 {
@@ -1805,8 +1812,11 @@ std::string gen_calc_kernel(const Plan& p, const std::vector<ColumnType>& cols, 
     // output (flag byte, then the compact row: GenSaveDataCode,
     // AriesExprCalcNode.cpp:76-108)
     const std::string OS = o.blocks ? "os_" : std::to_string(OB);
+    const int waves = calc_waves(p);
+    const std::string wv = std::to_string(waves);
+    const std::string waves_attr = waves ? "__attribute__((amdgpu_waves_per_eu(" + wv + ", " + wv + "))) " : "";
     E.os << "extern \"C\" __global__ void __launch_bounds__(" << T << ") "
-         << (calc_one_wave(p) ? "__attribute__((amdgpu_waves_per_eu(1, 1))) " : "") << name << "("
+         << waves_attr << name << "("
          << (o.blocks ? "IterArgs" : "ColArgs") << " a)\n{\n";
     emit_const_prologue(E, {p}, one_row);
     E.os << "  __shared__ u32 tile[(" << T << " * " << (o.blocks ? OB + 1 : OB) << " + 3) / 4];\n";
