@@ -861,10 +861,43 @@ template <int W> UPD_DEV Dec<W> ddiv_rt(const Dec<W>& a, const Dec<W>& b, u32 S,
     return r;
 }
 
+typedef unsigned int u32x4u __attribute__((vector_size(16), aligned(4)));
+typedef unsigned int u32x2u __attribute__((vector_size(8), aligned(4)));
+
+// Decode one compact DECIMAL row (decimal.cu:168-176): B little-endian bytes
+// at row*B, sign in bit 7 of the last byte.  Loads are the aligned dwords
+// covering the row; the last rows of a column, whose covering dwords would
+// run past the column, take a byte path.
+// *p, NT: read once (streamed past the caches)
+template <bool NT, class T> UPD_DEV T load_as(const T* p)
+{
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
+// N dwords from a 4-byte aligned address, by 16-byte loads
+template <int N, bool NT = true> UPD_DEV void load_dwords(const u32* p, u32* dw)
+{
+#pragma unroll
+    for (int i = 0; i + 4 <= N; i += 4) {
+        const u32x4u v = load_as<NT>(reinterpret_cast<const u32x4u*>(p + i));
+        dw[i] = v[0];
+        dw[i + 1] = v[1];
+        dw[i + 2] = v[2];
+        dw[i + 3] = v[3];
+    }
+    if constexpr ((N & 3) >= 2) {
+        const u32x2u v = load_as<NT>(reinterpret_cast<const u32x2u*>(p + (N & ~3)));
+        dw[N & ~3] = v[0];
+        dw[(N & ~3) + 1] = v[1];
+    }
+    if constexpr ((N & 1) != 0) dw[N - 1] = load_as<NT>(p + (N - 1));
+}
+
 // Decode one compact row of B bytes (B at run time) into W limbs.  The
 // caller guarantees the magnitude fits W limbs; when B > 4 W only the low
 // 4 W bytes and the sign byte are read.
-template <int W> UPD_DEV Dec<W> load_compact_rt(const u8* __restrict__ col, usize row, u32 B, usize colbytes)
+template <int W, bool NT = true> UPD_DEV Dec<W> load_compact_rt(const u8* __restrict__ col, usize row, u32 B, usize colbytes)
 {
     const usize off = row * (usize)B;
     const u32 nb = B < 4u * W ? B : 4u * W;
@@ -872,23 +905,28 @@ template <int W> UPD_DEV Dec<W> load_compact_rt(const u8* __restrict__ col, usiz
     const u32 sh = (u32)(off & 3u);
     const u32 nd = (sh + nb + 3u) >> 2;   // dwords covering the magnitude bytes
     u32 dw[W + 2];
-    const bool fast = (d0 + nd) * 4u <= colbytes;
     const u32* p = reinterpret_cast<const u32*>(col) + d0;
+    if ((d0 + W + 1) * 4u <= colbytes) {
+        // 16 bytes a load, as many as reach into the row
 #pragma unroll
-    for (int i = 0; i < W + 1; i++) {
-        u32 x = 0;
-        if ((u32)i < nd) {
-            if (fast) {
-                x = __builtin_nontemporal_load(p + i);
+        for (int i = 0; i < W; i += 4) {
+            if (i == 0 || (u32)i < nd) {
+                load_dwords<(W < 4 ? W : 4), NT>(p + i, dw + i);  // W is 2 or a multiple of 4
             } else {
 #pragma unroll
-                for (int b = 0; b < 4; b++) {
-                    const usize o = (d0 + (usize)i) * 4u + (usize)b;
-                    x |= (o < colbytes ? (u32)col[o] : 0u) << (8 * b);
-                }
+                for (int j = i; j < i + 4 && j < W; j++) dw[j] = 0u;
             }
         }
-        dw[i] = x;
+        dw[W] = (u32)W < nd ? load_as<NT>(p + W) : 0u;
+    } else {
+        // the column's last rows: whole dwords inside it, then the bytes of
+        // its partial last dword
+        const usize whole = colbytes >> 2;
+        u32 last = 0;
+        for (usize o = whole * 4u; o < colbytes; o++) last |= (u32)col[o] << (8u * (u32)(o & 3u));
+#pragma unroll
+        for (int i = 0; i < W + 1; i++)
+            dw[i] = (u32)i >= nd ? 0u : d0 + (usize)i < whole ? p[i] : (d0 + (usize)i == whole ? last : 0u);
     }
     dw[W + 1] = 0u;
     Dec<W> r;
@@ -1119,32 +1157,6 @@ template <int WO, int WA, int WB, int FAITH> UPD_DEV Dec<WO> dmod(const Dec<WA>&
 
 // ---------------------------------------------------------------- compact codec
 
-typedef unsigned int u32x4u __attribute__((vector_size(16), aligned(4)));
-typedef unsigned int u32x2u __attribute__((vector_size(8), aligned(4)));
-
-// Decode one compact DECIMAL row (decimal.cu:168-176): B little-endian bytes
-// at row*B, sign in bit 7 of the last byte.  Loads are the aligned dwords
-// covering the row; the last rows of a column, whose covering dwords would
-// run past the column, take a byte path.
-// N dwords from a 4-byte aligned address, by 16-byte loads
-template <int N> UPD_DEV void load_dwords(const u32* p, u32* dw)
-{
-#pragma unroll
-    for (int i = 0; i + 4 <= N; i += 4) {
-        const u32x4u v = __builtin_nontemporal_load(reinterpret_cast<const u32x4u*>(p + i));
-        dw[i] = v[0];
-        dw[i + 1] = v[1];
-        dw[i + 2] = v[2];
-        dw[i + 3] = v[3];
-    }
-    if constexpr ((N & 3) >= 2) {
-        const u32x2u v = __builtin_nontemporal_load(reinterpret_cast<const u32x2u*>(p + (N & ~3)));
-        dw[N & ~3] = v[0];
-        dw[(N & ~3) + 1] = v[1];
-    }
-    if constexpr ((N & 1) != 0) dw[N - 1] = __builtin_nontemporal_load(p + (N - 1));
-}
-
 // Decode the B-byte compact value at byte offset `off` of a 4-byte aligned
 // buffer of `colbytes` bytes (load_compact below: off = row * B; ALIGNED:
 // off is a multiple of 4).  The loads are 16 bytes wide: lanes are B bytes
@@ -1345,14 +1357,9 @@ template <int B, int W> UPD_DEV Mag<(B + 3) / 4> encode_compact(const Dec<W>& a)
 template <int AW, int W> UPD_DEV void acc_add(Mag<AW>& acc, const Dec<W>& v)
 {
     const u32 m = v.neg ? 0xffffffffu : 0u;
-    u64 c = v.neg ? 1u : 0u;
+    u32 c = v.neg ? 1u : 0u;
 #pragma unroll
-    for (int i = 0; i < AW; i++) {
-        u32 x = (i < W) ? (v.m.w[i] ^ m) : m;
-        u64 s = (u64)acc.w[i] + x + c;
-        acc.w[i] = (u32)s;
-        c = s >> 32;
-    }
+    for (int i = 0; i < AW; i++) acc.w[i] = addc(acc.w[i], i < W ? v.m.w[i] ^ m : m, c);
 }
 
 template <int AW> UPD_DEV void acc_merge(Mag<AW>& acc, const Mag<AW>& o)
