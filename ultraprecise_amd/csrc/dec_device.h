@@ -868,8 +868,21 @@ typedef unsigned int u32x2u __attribute__((vector_size(8), aligned(4)));
 // at row*B, sign in bit 7 of the last byte.  Loads are the aligned dwords
 // covering the row; the last rows of a column, whose covering dwords would
 // run past the column, take a byte path.
-// *p, NT: read once (streamed past the caches)
-template <bool NT, class T> UPD_DEV T load_as(const T* p)
+// four, two and one dwords from a 4-byte aligned address; NT: read once
+// (streamed past the caches)
+template <bool NT> UPD_DEV u32x4u load4(const u32* p)
+{
+    const u32x4u* q = reinterpret_cast<const u32x4u*>(p);
+    if constexpr (NT) return __builtin_nontemporal_load(q);
+    else return *q;
+}
+template <bool NT> UPD_DEV u32x2u load2(const u32* p)
+{
+    const u32x2u* q = reinterpret_cast<const u32x2u*>(p);
+    if constexpr (NT) return __builtin_nontemporal_load(q);
+    else return *q;
+}
+template <bool NT> UPD_DEV u32 load1(const u32* p)
 {
     if constexpr (NT) return __builtin_nontemporal_load(p);
     else return *p;
@@ -880,18 +893,18 @@ template <int N, bool NT = true> UPD_DEV void load_dwords(const u32* p, u32* dw)
 {
 #pragma unroll
     for (int i = 0; i + 4 <= N; i += 4) {
-        const u32x4u v = load_as<NT>(reinterpret_cast<const u32x4u*>(p + i));
+        const u32x4u v = load4<NT>(p + i);
         dw[i] = v[0];
         dw[i + 1] = v[1];
         dw[i + 2] = v[2];
         dw[i + 3] = v[3];
     }
     if constexpr ((N & 3) >= 2) {
-        const u32x2u v = load_as<NT>(reinterpret_cast<const u32x2u*>(p + (N & ~3)));
+        const u32x2u v = load2<NT>(p + (N & ~3));
         dw[N & ~3] = v[0];
         dw[(N & ~3) + 1] = v[1];
     }
-    if constexpr ((N & 1) != 0) dw[N - 1] = load_as<NT>(p + (N - 1));
+    if constexpr ((N & 1) != 0) dw[N - 1] = load1<NT>(p + (N - 1));
 }
 
 // Decode one compact row of B bytes (B at run time) into W limbs.  The
@@ -917,7 +930,7 @@ template <int W, bool NT = true> UPD_DEV Dec<W> load_compact_rt(const u8* __rest
                 for (int j = i; j < i + 4 && j < W; j++) dw[j] = 0u;
             }
         }
-        dw[W] = (u32)W < nd ? load_as<NT>(p + W) : 0u;
+        dw[W] = (u32)W < nd ? load1<NT>(p + W) : 0u;
     } else {
         // the column's last rows: whole dwords inside it, then the bytes of
         // its partial last dword
