@@ -50,3 +50,17 @@ extern "C" int divmod_run(int nx, int nb, const uint32_t* X, const uint32_t* B, 
 }
 
 extern "C" uint32_t recip2_run(uint32_t d1, uint32_t d0) { return recip_2word(d1, d0); }
+
+// x / y with the reference's path quirks at S = 24, one row
+extern "C" void ddiv_run(uint32_t a, uint32_t aneg, const uint32_t* b, uint32_t bneg, uint32_t* out)
+{
+    Dec<1> x;
+    Dec<3> y;
+    x.m.w[0] = a;
+    x.neg = aneg;
+    memcpy(y.m.w, b, sizeof y.m.w);
+    y.neg = bneg;
+    const Dec<4> r = ddiv<4, 1, 3, 24, 1>(x, y);
+    memcpy(out, r.m.w, sizeof r.m.w);
+    out[4] = r.neg;
+}

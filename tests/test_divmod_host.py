@@ -68,3 +68,15 @@ def test_two_word_reciprocal(lib):
         d1 = tops[i % 8] if i % 8 < 4 else rng.getrandbits(31) | 0x80000000
         d0 = _word(rng)
         assert lib.recip2_run(ctypes.c_uint32(d1), ctypes.c_uint32(d0)) == ((1 << 96) - 1) // (d1 << 32 | d0) - (1 << 32)
+
+
+@pytest.mark.parametrize("bits", [1, 31, 32, 33, 63, 64, 65, 96])
+@pytest.mark.parametrize("signs", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_zero_dividend_is_plus_zero(lib, bits, signs):
+    """also where the reference's bisection would return 1: a divisor of up
+    to 64 bits against a dividend of none"""
+    b = np.array(_words((1 << bits) - 1, 3), dtype=np.uint32)
+    out = np.zeros(5, dtype=np.uint32)
+    lib.ddiv_run(ctypes.c_uint32(0), ctypes.c_uint32(signs[0]), b.ctypes.data_as(ctypes.c_void_p),
+                 ctypes.c_uint32(signs[1]), out.ctypes.data_as(ctypes.c_void_p))
+    assert not out.any()

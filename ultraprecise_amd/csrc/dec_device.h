@@ -821,7 +821,7 @@ template <int W> UPD_DEV Dec<W> ddiv_rt(const Dec<W>& a, const Dec<W>& b, u32 S,
         const u32 bla = bitlen(a.m), blb = bitlen(bs), blx = bitlen(X);
         path_i = !bzero && bla + (u32)est_shift_bits((int)S) - 1u <= 64u && blb <= 64u;
         path_ii = !path_i && blb <= 32u;
-        path_iii_one = !path_i && !path_ii && blx < blb && blb - blx <= 64u;
+        path_iii_one = !path_i && !path_ii && !azero && blx < blb && blb - blx <= 64u;
     }
     Mag<W + 1> Q;
     Mag<W> Rn, vn, T;
@@ -1076,7 +1076,7 @@ UPD_DEV Dec<WO> ddiv(const Dec<WA>& a, const Dec<WB>& b, u32* err = nullptr)
         const u32 bla = bitlen(a.m), blb = bitlen(bs), blx = bitlen(X);
         path_i = !bzero && bla + (u32)est_shift_bits(S) - 1u <= 64u && blb <= 64u;
         path_ii = !path_i && blb <= 32u;
-        path_iii_one = !path_i && !path_ii && blx < blb && blb - blx <= 64u;
+        path_iii_one = !path_i && !path_ii && !azero && blx < blb && blb - blx <= 64u;
     }
     Mag<WX + 1> Q;
     Mag<WB> Rn, vn, T;
