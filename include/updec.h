@@ -377,9 +377,10 @@ int updec_module_cache_stats(int64_t* rtc_compiles, int64_t* memory_hits, int64_
  * updec_expr_compile does, then build a register program.  Every register
  * holds W limbs, W in {2, 4, 8, 16, 32, 64, 128, 256, 512} the smallest
  * that holds every intermediate exactly; UPDEC_EUNSUPPORTED when none does.
- * Up to 32 limbs one lane holds a value; the 64- to 512-limb classes
- * (extended-mode programs only) spread a value over a group of lanes (the
- * reference's multi-lane XMP form, AriesExprCalcNode.cpp:1320-1400).
+ * Up to 32 limbs values lie in registers; those of the 64- to 512-limb
+ * classes (extended-mode programs only) in a workspace that the batch object
+ * holds (at most 1 GiB, or 64 rows' worth where that is more; allocated when
+ * the first such query is added and grown by later ones).
  *
  * A batch collects queries (program, device columns, rows, output image and
  * count) and runs them with one set of launches: persistent kernels per
@@ -397,12 +398,14 @@ int updec_vm_info(updec_vm_t v, int32_t* width, int32_t* nins, int32_t* nregs, i
 int updec_vm_listing(updec_vm_t v, char* buf, size_t cap, size_t* needed);
 void updec_vm_free(updec_vm_t v);
 int updec_batch_create(int32_t max_queries, int32_t max_items, updec_batch_t* out);
-/* per width class (0..4 for W = 2..32): rows per work item and resident
- * blocks per compute unit of the persistent kernel */
+/* per width class: rows per work item and resident blocks per compute unit
+ * of the persistent kernel (0..4 for W = 2..32; the classes from 5 on share
+ * one kernel, whose blocks are single waves and as many as the largest of
+ * their settings asks for) */
 int updec_batch_tuning(updec_batch_t b, int32_t width_class, int64_t rows_per_item, int32_t blocks_per_cu);
-/* lanes per value of a multi-lane class (width_class 5..8, W = 64 .. 512
- * limbs): W / 4 (4 limbs per lane, the default) or W / 8 (8 limbs per lane),
- * at most 64 (the 512-limb class: 64 lanes of 8 limbs) */
+/* lanes per value of a wide class (width_class 5..8, W = 64 .. 512 limbs):
+ * W / 4 or W / 8, at most 64.  Checked and accepted; every value lies in one
+ * lane's part of the workspace, so it changes nothing. */
 int updec_batch_lanes(updec_batch_t b, int32_t width_class, int32_t lanes);
 /* *index_out (optional): the query's position in the pending batch.
  * UPDEC_EFULL (nothing staged) when the batch's query, work-item or program

@@ -1,31 +1,26 @@
 """Autotuner for the interpreter's persistent kernels.
 
-Per register-width class (W = 2 .. 32 limbs one value per lane, W = 64 ..
-512 limbs one value per group of lanes) it times representative queries of
-that width -- seeded serving queries whose programs land in the class --
-over every candidate (rows per work item, resident blocks per compute unit,
-and for the multi-lane classes lanes per value: W / 4 or W / 8, at most 64)
-and keeps the fastest.  Results are cached per device name in a JSON file
+Per register-width class (W = 2 .. 32 limbs in registers, W = 64 .. 512 limbs
+in a workspace) it times representative queries of that width -- seeded
+serving queries whose programs land in the class -- over every candidate
+(rows per work item, resident blocks per compute unit; a block of the wide
+classes is one wave) and keeps the fastest.  Results are cached per device name in a JSON file
 so a process pays the search once.
 """
 import json
 import os
 
 DEFAULT_CANDIDATES = ((1024, 4), (2048, 4), (4096, 2), (4096, 4), (8192, 4), (8192, 8), (16384, 4), (32768, 4))
-MULTI_LANE_ITEMS = ((128, 4), (256, 4), (512, 4), (512, 8), (1024, 4), (1024, 8), (2048, 4))
+WIDE_ITEMS = ((64, 16), (128, 16), (256, 8), (256, 16), (512, 16), (1024, 16))
 
 
 def class_rows(width, rows):
     """rows timed per query of a class: fewer for the costly wide classes"""
-    return rows if width <= 32 else max(20_000, rows * 32 // (width * 8))
+    return rows if width <= 32 else max(100_000, rows * 32 // (width * 2))
 
 
 def candidates_for(U, cls, candidates):
-    w = U.VM_CLASS_WIDTHS[cls]
-    if cls < U.VM_FIRST_MULTI_LANE:
-        return [(rpi, bpc) for rpi, bpc in candidates]
-    lanes = sorted({min(64, w // 4), w // 8})
-    return [(rpi, bpc, ln) for rpi, bpc in MULTI_LANE_ITEMS for ln in lanes if ln <= 64]
+    return list(candidates if cls < U.VM_FIRST_MULTI_LANE else WIDE_ITEMS)
 
 
 def cache_path(device_name):
@@ -51,7 +46,7 @@ def representative_queries(U, W, per_class=2, seed=77, max_draws=12000):
 
 
 def tune(U, rows=2_000_000, candidates=DEFAULT_CANDIDATES, reps=3, use_cache=True):
-    """returns {class: (rows_per_item, blocks_per_cu[, lanes per value])}"""
+    """returns {class: (rows_per_item, blocks_per_cu)}"""
     from . import workloads as W
     name = U.device_info()["name"]
     path = cache_path(name)
@@ -74,7 +69,7 @@ def tune(U, rows=2_000_000, candidates=DEFAULT_CANDIDATES, reps=3, use_cache=Tru
         best = None
         for cand in candidates_for(U, cls, candidates):
             b = U.Batch(max_queries=len(qs), max_items=1 << 16)
-            b.tune(cls, cand[0], cand[1], lanes=cand[2] if len(cand) > 2 else None)
+            b.tune(cls, cand[0], cand[1])
 
             def launch():
                 for k, (p, c) in enumerate(zip(progs, cols)):

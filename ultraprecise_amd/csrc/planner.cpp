@@ -3,6 +3,7 @@
 #include "planner.h"
 
 #include <algorithm>
+#include <array>
 #include <cctype>
 #include <cstdio>
 #include <cstdlib>
@@ -2583,6 +2584,142 @@ struct VmBuilder {
 
 }  // namespace
 
+// The workspace form of a finished program (vm_wide.h): every value gets a
+// row range by its own bound, not the class width, reused when its last
+// reader is past, and a slot of the kernel's table.
+static bool build_wide_program(VmProgram* pr, const std::vector<ColumnType>& cols, std::string* err)
+{
+    using namespace updec_vm;
+    struct Value {
+        int bits = 1, slot = 0;
+        uint32_t row = 0, rows = 0;
+        size_t last = 0;   // last instruction that reads it
+    };
+    const size_t n = pr->ins.size();
+    std::vector<Value> val(n);
+    // readers: which value each register holds when it is read
+    std::vector<int> reg(kMaxRegs, -1);
+    std::vector<std::array<int, 2>> from(n, {-1, -1});
+    uint32_t colmask = 0;
+    for (size_t i = 0; i < n; i++) {
+        const Ins& I = pr->ins[i];
+        const bool binary = I.op >= OP_ADD && I.op <= OP_DIV;
+        for (int k = 0; k < (binary ? 2 : 1); k++) {
+            const Operand& o = k ? I.b : I.a;
+            if (o.kind == K_COL) colmask |= 1u << o.idx;
+            if (o.kind == K_REG) from[i][k] = reg[o.idx];
+            if (o.kind == K_LAST) from[i][k] = (int)i - 1;
+            if (from[i][k] >= 0) val[(size_t)from[i][k]].last = i;
+        }
+        if (I.dst != kNoStore) reg[I.dst] = (int)i;
+    }
+    const int root = pr->root == kNoStore ? (int)n - 1 : reg[pr->root];
+    if (root != (int)n - 1) { *err = "internal: the root is not the last result"; return false; }
+    uint32_t top = 0, colrow[kMaxCols] = {};
+    for (int c = 0; c < kMaxCols && c < (int)cols.size(); c++)
+        if ((colmask >> c) & 1u) {
+            colrow[c] = top;
+            top += (uint32_t)(compact_bytes(cols[c].P) + 3) / 4;
+        }
+    const uint32_t first = top;
+    auto rows_of = [](int bits) { return (uint32_t)words_for(bits) + 2u; };
+    uint32_t ru = 1, rv = 1;
+    std::vector<uint32_t> words(wide::kHead, 0u);
+    for (size_t i = 0; i < n; i++) {
+        const Ins& I = pr->ins[i];
+        const bool binary = I.op >= OP_ADD && I.op <= OP_DIV;
+        int b[2] = {1, 1};
+        uint32_t ow[2] = {0, 0};
+        for (int k = 0; k < (binary ? 2 : 1); k++) {
+            const Operand& o = k ? I.b : I.a;
+            if (o.kind == K_COL) {
+                // what a row can hold, not the column's statistic: the
+                // workspace has to fit whatever the data are
+                b[k] = 8 * compact_bytes(cols[o.idx].P) - 1;
+                ow[k] = o.idx;
+            } else if (o.kind == K_CONST) {
+                b[k] = 1;
+                const uint32_t* c = pr->consts.data() + (size_t)o.idx * (size_t)(pr->W + 1);
+                for (int w = pr->W; w > 0 && b[k] == 1; w--)
+                    if (c[w]) b[k] = 32 * w;
+                ow[k] = o.idx | 0x100u;
+            } else {
+                b[k] = val[(size_t)from[i][k]].bits;
+                ow[k] = (uint32_t)val[(size_t)from[i][k]].slot;
+            }
+        }
+        uint32_t sa = 0, arg = 0;
+        int bits = b[0];
+        switch (I.op) {
+        case OP_ADD:
+        case OP_SUB: {
+            sa = I.a.shift;
+            arg = I.b.shift;
+            const int xa = b[0] + (sa ? pow10_bits((int)sa) : 0), xb = b[1] + (arg ? pow10_bits((int)arg) : 0);
+            if (sa && arg) { *err = "internal: both operands of a sum aligned"; return false; }
+            bits = std::max(xa, xb) + 1;
+            break;
+        }
+        case OP_MUL: bits = b[0] + b[1]; break;
+        case OP_DIV:
+            sa = I.arg;
+            bits = b[0] + pow10_bits(I.arg) + 1;
+            if (words_for(b[1]) > 32) ru = std::max(ru, rows_of(bits) + rows_of(b[1]));
+            rv = std::max(rv, rows_of(b[1]));
+            break;
+        case OP_UP:
+            arg = I.arg;
+            bits = b[0] + pow10_bits(I.arg);
+            break;
+        case OP_DOWN:
+            arg = I.arg;
+            bits = std::max(1, b[0] - (pow10_bits(I.arg) - 1));
+            break;
+        default: break;
+        }
+        // the lowest rows and the first slot that no live value has
+        Value& v = val[i];
+        v.bits = bits;
+        v.rows = rows_of(std::max(bits, b[0]));   // OP_DOWN's passes start at the argument's width
+        if (i + 1 == n) v.last = n;
+        uint32_t at = first, slots = 0;
+        for (bool moved = true; moved;) {
+            moved = false;
+            for (size_t k = 0; k < i; k++)
+                if (val[k].last >= i && at < val[k].row + val[k].rows && val[k].row < at + v.rows) {
+                    at = val[k].row + val[k].rows;
+                    moved = true;
+                }
+        }
+        for (size_t k = 0; k < i; k++)
+            if (val[k].last >= i) slots |= 1u << val[k].slot;
+        v.slot = kMaxCols;
+        while (v.slot < (int)wide::kSlots && ((slots >> v.slot) & 1u)) v.slot++;
+        if (v.slot == (int)wide::kSlots || at + v.rows >= 1u << 20) { *err = "expression needs too large a workspace"; return false; }
+        v.row = at;
+        top = std::max(top, at + v.rows);
+        words.push_back((uint32_t)I.op | ((uint32_t)v.slot << 4) | (at << 12));
+        words.push_back(ow[0] | (sa << 16));
+        words.push_back(ow[1] | (arg << 16));
+    }
+    auto take = [&](uint32_t rows) {
+        const uint32_t r = top;
+        top += rows;
+        return r;
+    };
+    const uint32_t acc = (uint32_t)std::min((8 * pr->outB + 31) / 32, words_for(val[n - 1].bits) + 1) + 2u;
+    words[wide::kHeadU] = take(ru);
+    words[wide::kHeadV] = take(rv);
+    words[wide::kHeadPos] = take(acc);
+    words[wide::kHeadNeg] = take(acc);
+    words[wide::kHeadAcc] = acc;
+    words[wide::kHeadCols] = colmask;
+    for (int c = 0; c < kMaxCols; c++) words[wide::kHeadCol + (uint32_t)c] = colrow[c];
+    pr->wide = std::move(words);
+    pr->wide_rows = top;
+    return true;
+}
+
 bool build_vm_program(const Plan& p, const std::vector<ColumnType>& cols, VmProgram* out, std::string* err)
 {
     VmProgram prog;
@@ -2657,6 +2794,7 @@ bool build_vm_program(const Plan& p, const std::vector<ColumnType>& cols, VmProg
         *err = "expression needs more interpreter registers than its width class holds";
         return false;
     }
+    if (updec_vm::runs_wide(prog.wclass, prog.faithful) && !build_wide_program(&prog, cols, err)) return false;
     *out = std::move(prog);
     return true;
 }

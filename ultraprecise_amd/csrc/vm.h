@@ -35,16 +35,16 @@ constexpr uint8_t kNoStore = 0xff;
 constexpr int kMaxRegs = 8;
 constexpr int kMaxCols = 8;
 constexpr int kMaxIns = 512;
-// W = 2 .. 32: one value per lane; W = 64 .. 512: one value per group of
-// lanes (dec_mlane.h), L limbs per lane, for extended-mode programs whose
-// exact intermediates need more than 32 limbs
+// W = 2 .. 32: values in registers of the class width; W = 64 .. 512, for
+// extended-mode programs whose exact intermediates need more than 32 limbs:
+// values in memory at the limbs they have (vm_wide.h)
 constexpr int kNumClasses = 9;
 constexpr int kFirstMultiLane = 5;
 constexpr int kClassW[kNumClasses] = {2, 4, 8, 16, 32, 64, 128, 256, 512};
 constexpr int kMaxAccWords = 514;               // accumulator limbs of the widest class (W + 2)
-// registers per class: the register file is held in LDS, so the wide
-// one-value-per-lane classes get fewer registers to keep four blocks
-// resident per CU; a multi-lane register is L + 1 words per lane
+// registers per class: up to 32 limbs the register file is held in LDS, so
+// the wider of these classes get fewer registers to keep four blocks
+// resident per CU
 constexpr int kClassRegs[kNumClasses] = {8, 8, 8, 6, 4, 8, 8, 8, 8};
 
 struct Operand {
@@ -59,6 +59,26 @@ struct Ins {
     uint16_t arg;
     Operand a, b;
 };
+
+// Programs of these classes run on the kernel of vm_wide.h
+constexpr bool runs_wide(int wclass, bool faithful) { return wclass >= kFirstMultiLane && !faithful; }
+
+// The form of a program that vm_wide.h evaluates (planner.cpp,
+// build_wide_program): a header of kHead words, then kIns words an
+// instruction,
+//   op | slot << 4 | row << 12
+//   operand a | shift << 16   (the scale argument of a division)
+//   operand b | shift << 16   (the argument of OP_UP and OP_DOWN)
+// with operands slot or constant index | constant? << 8.  A slot names a
+// value while it is live (columns are slots 0 .. 7); rows are limbs of the
+// wave's workspace.
+namespace wide {
+constexpr uint32_t kHead = 18, kIns = 3, kSlots = 32;
+// header words: rows of a division's dividend and divisor (where they are
+// held in memory), of the two accumulators and their length; mask of the
+// columns read; from kHeadCol on each column's row
+constexpr uint32_t kHeadU = 0, kHeadV = 1, kHeadPos = 2, kHeadNeg = 3, kHeadAcc = 4, kHeadCols = 5, kHeadCol = 6;
+}  // namespace wide
 
 // One query of a batch.  Constants are stored at the query's class width as
 // W + 1 words {sign, limbs...} starting at const_off.
@@ -89,6 +109,9 @@ struct Item {
 // Device-resident batch header: per class item ranges and the work counters
 // the persistent kernels take items from.
 struct Header {
+    uint8_t* workspace;          // of the wide kernel: `stride` bytes for each of `wide_blocks` blocks
+    uint64_t stride;
+    uint32_t wide_blocks;
     uint32_t nqueries;
     uint32_t class_item0[kNumClasses];
     uint32_t class_nitems[kNumClasses];

@@ -22,10 +22,10 @@
 #include "../../include/updec.h"
 #include "api_internal.h"
 #include "dec_device.h"
-#include "dec_mlane.h"
 #include "planner.h"
 #include "vm.h"
 #include "vm_device.h"
+#include "vm_wide.h"
 
 using namespace updec;
 using namespace updec_vm;
@@ -38,11 +38,11 @@ namespace {
         if (e_ != hipSuccess) return api_fail(UPDEC_EHIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-constexpr int kBlock[kNumClasses] = {256, 256, 128, 64, 64, 128, 128, 128, 128};
+constexpr int kBlock[kFirstMultiLane] = {256, 256, 128, 64, 64};
 
 template <int W> constexpr int class_of()
 {
-    return W == 2 ? 0 : W == 4 ? 1 : W == 8 ? 2 : W == 16 ? 3 : W == 32 ? 4 : W == 64 ? 5 : W == 128 ? 6 : W == 256 ? 7 : 8;
+    return W == 2 ? 0 : W == 4 ? 1 : W == 8 ? 2 : W == 16 ? 3 : 4;
 }
 
 template <int W, int T>
@@ -104,127 +104,38 @@ __global__ void __launch_bounds__(T)
     }
 }
 
-// ---------------------------------------------------------------- multi-lane classes
+// ---------------------------------------------------------------- wide classes
 
-// the lane's slice of register i: L limbs and the sign, in LDS at
-// [register][word][lane] like RegFile
-template <int L, int STRIDE> struct MLRegFile {
-    u32* base;
-    UPD_DEV ml::MDec<L> get(u32 i) const
-    {
-        const u32* p = base + i * (u32)((L + 1) * STRIDE);
-        ml::MDec<L> r;
-#pragma unroll
-        for (int w = 0; w < L; w++) r.m.w[w] = p[w * STRIDE];
-        r.neg = p[L * STRIDE];
-        return r;
-    }
-    UPD_DEV void set(u32 i, const ml::MDec<L>& v)
-    {
-        u32* p = base + i * (u32)((L + 1) * STRIDE);
-#pragma unroll
-        for (int w = 0; w < L; w++) p[w * STRIDE] = v.m.w[w];
-        p[L * STRIDE] = v.neg;
-    }
-};
-
-template <int L, int TPI, class RF>
-UPD_DEV ml::MDec<L> fetch_ml(u32 ow, const Query* q, const u32* cst, const RF& R, const ml::MDec<L>& last, usize row,
-                             const ml::Grp<TPI>& g)
+// Persistent kernel of the classes of 64 limbs and more (vm_wide.h): a block
+// is one wave, an item's rows are taken 64 at a time, one lane each, with
+// every value in the block's workspace.
+//
+// What bounds it: latency of the workspace's loads (a value's limb is one
+// 256-byte line; three quarters of them hit L2) and integer issue, 40 % of the
+// time at twelve waves a CU.  The form it replaced spread every value over 16
+// to 64 lanes at the program's worst-case width.  2 M rows of
+// "((((c-c)*a)*((a/c)*(c/a)))+(b+((b/(a-a))/c)))" at DECIMAL(300,100), a
+// 256-limb program: 5.1 ms (11.6 at two waves a CU, 7.4 at four, 5.6 at
+// eight); 9 M rows 310 -> 19 ms, 2.2 M rows of a 64-limb program at
+// DECIMAL(76,25) 15.7 -> 2.0, 28,000 rows of a 128-limb one 3.4 -> 0.15.
+constexpr u32 kSumLimbs = 512;   // of the accumulators at a time
+__global__ void __launch_bounds__(64, 3)
+    k_vm_sum_wide(Header* h, const Query* qs, const u32* prog, const u32* cst, const Item* items, u32* partials)
 {
-    constexpr int W = L * TPI;
-    const u32 kind = ow & 0xffu, idx = (ow >> 8) & 0xffu, shift = ow >> 16;
-    ml::MDec<L> v;
-    if (kind == K_LAST) {
-        v = last;
-    } else if (kind == K_REG) {
-        v = R.get(idx);
-    } else if (kind == K_COL) {
-        const u32 B = q->colbytes[idx];
-        v = ml::load_compact<L, TPI>(q->col[idx], row, B, (usize)q->rows * B, g);
-    } else {
-        // constants at the class width: {sign, W limbs}
-        const u32* k = cst + idx * (u32)(W + 1);
-        v.neg = k[0];
-#pragma unroll
-        for (int w = 0; w < L; w++) v.m.w[w] = k[1 + g.rank * L + w];
-    }
-    if (shift) ml::mul_p10<L, TPI>(v.m, shift, g);
-    return v;
-}
-
-// the register program of one row, evaluated by the row's group of TPI lanes
-// (extended mode: multi-lane classes hold no faithful programs)
-template <int L, int TPI, class RF>
-UPD_DEV ml::MDec<L> vm_eval_ml(const Query* q, const u32* prog, const u32* cst, usize row, RF& R, const ml::Grp<TPI>& g)
-{
-    const u32 n = q->nins;
-    ml::MDec<L> last;
-    last.m = ml::mzero<L>();
-    last.neg = 0u;
-    for (u32 pc = 0; pc < n; pc++) {
-        const u32 w0 = prog[3 * pc], w1 = prog[3 * pc + 1], w2 = prog[3 * pc + 2];
-        const u32 op = w0 & 0xffu, dst = (w0 >> 8) & 0xffu, arg = w0 >> 16;
-        const ml::MDec<L> a = fetch_ml<L, TPI, RF>(w1, q, cst, R, last, row, g);
-        ml::MDec<L> r;
-        if (op == OP_MOV) {
-            r = a;
-        } else if (op == OP_NEG) {
-            r = a;
-            r.neg ^= 1u;
-        } else if (op == OP_UP) {
-            r = a;
-            ml::mul_p10<L, TPI>(r.m, arg, g);
-        } else if (op == OP_DOWN) {
-            r = a;
-            ml::div_p10<L, TPI>(r.m, arg, g);
-        } else {
-            const ml::MDec<L> b = fetch_ml<L, TPI, RF>(w2, q, cst, R, last, row, g);
-            if (op == OP_ADD) {
-                r = ml::add<L, TPI>(a, b, g);
-            } else if (op == OP_SUB) {
-                r = ml::sub<L, TPI>(a, b, g);
-            } else if (op == OP_MUL) {
-                r.m = ml::mul<L, TPI>(a.m, b.m, g);
-                r.neg = a.neg ^ b.neg;
-            } else {
-                r = ml::div<L, TPI>(a, b, arg, g);
-            }
-        }
-        if (dst != kNoStore) R.set(dst, r);
-        last = r;
-    }
-    return q->root == kNoStore ? last : R.get(q->root);
-}
-
-// Persistent kernel of a multi-lane class: blocks take work items as
-// k_vm_sum does; within an item the block's T / TPI groups take rows in
-// turn, each group evaluating its row's program and folding the stored
-// value into its two's complement accumulator; the block then adds its
-// groups' accumulators column by column and writes the item's partial.
-template <int L, int TPI, int T>
-__global__ void __launch_bounds__(T)
-    k_vm_sum_ml(Header* h, const Query* qs, const u32* prog, const u32* cst, const Item* items, u32* partials)
-{
-    constexpr int W = L * TPI;
-    constexpr int CLS = class_of<W>();
-    constexpr int AW = W + 2;
-    constexpr int NG = T / TPI;
     __shared__ u32 s_item;
-    __shared__ u32 regs[kClassRegs[CLS] * (L + 1) * T];
-    __shared__ u32 gacc[NG * AW];
-    __shared__ u64 csum[AW];
-    const u32 tid = threadIdx.x;
-    const ml::Grp<TPI> g;
-    const u32 grp = tid / (u32)TPI;
-    MLRegFile<L, T> R{regs + tid};
-    const u32 n = h->class_nitems[CLS];
-    const u32 i0 = h->class_item0[CLS];
+    __shared__ wide::Slots slots;
+    __shared__ i64 csum[kSumLimbs];
+    const u32 lane = threadIdx.x;
+    if (blockIdx.x >= h->wide_blocks) return;
+    u8* const ws = h->workspace + (usize)blockIdx.x * (usize)h->stride;
+    u32 n = 0;
+    for (int c = kFirstMultiLane; c < kNumClasses; c++) n += h->class_nitems[c];
+    const u32 i0 = h->class_item0[kFirstMultiLane];
     for (;;) {
         // as in k_vm_sum: the barrier keeps thread 0's item fetch apart from
         // its partial write of the previous iteration
         __syncthreads();
-        if (tid == 0) s_item = atomicAdd(&h->counter[CLS], 1u);
+        if (lane == 0) s_item = atomicAdd(&h->counter[kFirstMultiLane], 1u);
         __syncthreads();
         const u32 it = __builtin_amdgcn_readfirstlane(s_item);
         if (it >= n) break;
@@ -232,58 +143,96 @@ __global__ void __launch_bounds__(T)
         const Query* q = qs + I.query;
         const u32* qp = prog + 3u * q->ins_off;
         const u32* qc = cst + q->const_off;
-        const u32 ob = q->outB;
-        ml::Acc<L> acc = ml::acc_zero<L>();
-        for (usize row = I.row0 + grp; row < I.row1; row += NG) {
-            const ml::MDec<L> v = vm_eval_ml<L, TPI>(q, qp, qc, row, R, g);
-            ml::acc_add<L, TPI>(acc, ml::stored<L, TPI>(v, ob, g), g);
+        const u32 W = (u32)kClassW[0] << q->wclass;
+        const u32 na = wide::kword(qp, wide::kHeadAcc);
+        const u32 off = 4u * lane;
+        const wide::Dst pos{ws + (usize)wide::kword(qp, wide::kHeadPos) * wide::kRow, off};
+        const wide::Dst neg{ws + (usize)wide::kword(qp, wide::kHeadNeg) * wide::kRow, off};
+        for (u32 i = 0; i < na; i++) {
+            pos.put(i, 0u);
+            neg.put(i, 0u);
         }
+        for (usize r0 = I.row0; r0 < I.row1; r0 += 64u) {
+            // lanes past the item's end repeat its last row, uncounted
+            const bool active = r0 + lane < I.row1;
+            u32 sign;
+            const wide::Src v = wide::eval(q, qp, qc, W, ws, &slots, active ? r0 + lane : I.row1 - 1u, sign);
+            wide::accumulate(v, sign, active, q->outB, pos, neg);
+        }
+        __syncthreads();
+        // limb by limb over the lanes, then a carry pass
+        u32* dst = partials + (usize)(i0 + it) * kMaxAccWords;
+        i64 c = 0;
+        for (u32 w0 = 0; w0 < na; w0 += kSumLimbs) {
+            const u32 m = na - w0 < kSumLimbs ? na - w0 : kSumLimbs;
+            for (u32 w = lane; w < m; w += 64u) {
+                const u32* a = reinterpret_cast<const u32*>(pos.b + (usize)(w0 + w) * wide::kRow);
+                const u32* b = reinterpret_cast<const u32*>(neg.b + (usize)(w0 + w) * wide::kRow);
+                i64 s = 0;
+                for (u32 k = 0; k < 64u; k += 4u) {
+                    u32 x[4], y[4];
+                    load_dwords<4, false>(a + k, x);
+                    load_dwords<4, false>(b + k, y);
 #pragma unroll
-        for (int w = 0; w < L; w++) gacc[grp * AW + g.rank * L + w] = acc.m.w[w];
-        if (g.rank == TPI - 1) {
-            gacc[grp * AW + W] = acc.x0;
-            gacc[grp * AW + W + 1] = acc.x1;
-        }
-        __syncthreads();
-        for (u32 w = tid; w < (u32)AW; w += T) {
-            u64 s = 0;
-            for (u32 k = 0; k < (u32)NG; k++) s += gacc[k * AW + w];
-            csum[w] = s;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            u32* dst = partials + (usize)(i0 + it) * kMaxAccWords;
-            u64 c = 0;
-            for (int w = 0; w < AW; w++) {
-                const u64 t = csum[w] + c;
-                dst[w] = (u32)t;
+                    for (int t = 0; t < 4; t++) s += (i64)x[t] - (i64)y[t];
+                }
+                csum[w] = s;
+            }
+            __syncthreads();
+            // every lane follows the carries, lane 0 writes
+            for (u32 w = 0; w < m; w++) {
+                const i64 t = csum[w] + c;
+                if (lane == 0 && w0 + w < W + 2u) dst[w0 + w] = (u32)t;
                 c = t >> 32;
             }
+            __syncthreads();
         }
+        for (u32 w = na + lane; w < W + 2u; w += 64u) dst[w] = (u32)c;
     }
 }
 
-// SUM image and COUNT of a query of a multi-lane class: its items'
-// partials added column by column (64-bit words, no carries), then one
-// carry pass; the image keeps the low 32 limbs of the magnitude
-template <int AW> __device__ void final_query_wide(const Query* q, const u32* partials)
+// SUM image and COUNT of every query: one block each.  Lanes take the words
+// of the items' partials (consecutive words of an item, as many items at once
+// as fit a wave), waves take items in turn; the words are added without
+// carries as 64-bit sums, then one carry pass, and the image gets the low 32
+// limbs of the magnitude.
+//
+// What bounds it: latency of the partials' loads.  With one wave per query,
+// walking the items one after the other, 7,800 partials of a 256-limb query
+// took 6 ms, now 0.1.
+constexpr int kFinalThreads = 1024, kFinalAhead = 4;
+__global__ void __launch_bounds__(kFinalThreads) k_vm_final(const Header* h, const Query* qs, const u32* partials)
 {
-    __shared__ u64 cs[AW];
-    __shared__ u32 mag[AW];
-    for (u32 w = threadIdx.x; w < (u32)AW; w += 64) {
+    __shared__ u64 cs[kMaxAccWords];
+    const u32 qi = blockIdx.x, tid = threadIdx.x;
+    if (qi >= h->nqueries) return;
+    const Query* q = qs + qi;
+    const u32 aw = ((u32)kClassW[0] << q->wclass) + 2u;
+    for (u32 w = tid; w < aw; w += kFinalThreads) cs[w] = 0;
+    __syncthreads();
+    // words a row of lanes takes of one item, and the rows of the block
+    u32 wide = 4;
+    while (wide < aw && wide < 64u) wide <<= 1;
+    const u32 rows = kFinalThreads / wide, row = tid / wide;
+    const u32* base = partials + (usize)q->item0 * kMaxAccWords;
+    for (u32 w = tid % wide; w < aw; w += wide) {
         u64 s = 0;
-        for (u32 k = 0; k < q->nitems; k++) s += partials[(usize)(q->item0 + k) * kMaxAccWords + w];
-        cs[w] = s;
+        for (u32 k = row; k < q->nitems; k += rows * kFinalAhead) {
+#pragma unroll
+            for (u32 t = 0; t < (u32)kFinalAhead; t++)
+                if (k + t * rows < q->nitems) s += base[(usize)(k + t * rows) * kMaxAccWords + w];
+        }
+        if (s) atomicAdd(reinterpret_cast<unsigned long long*>(&cs[w]), (unsigned long long)s);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         u64 c = 0;
-        for (int w = 0; w < AW; w++) {
+        for (u32 w = 0; w < aw; w++) {
             const u64 t = cs[w] + c;
-            mag[w] = (u32)t;
+            cs[w] = (u32)t;
             c = t >> 32;
         }
-        const bool neg = (mag[AW - 1] >> 31) != 0;
+        const bool neg = ((u32)cs[aw - 1u] >> 31) != 0u;
         // magnitude of the two's complement value
         u64 cc = neg ? 1u : 0u;
         const u32 fm = neg ? 0xffffffffu : 0u;
@@ -293,8 +242,8 @@ template <int AW> __device__ void final_query_wide(const Query* q, const u32* pa
         o[2] = (u8)(q->outP & 0xffu);
         o[3] = (u8)(q->outS & 0xffu);
         o[4] = 0;
-        for (int w = 0; w < 32; w++) {
-            const u64 t = (u64)(mag[w] ^ fm) + cc;
+        for (u32 w = 0; w < 32u; w++) {
+            const u64 t = (u64)(w < aw ? (u32)cs[w] ^ fm : 0u) + (w < aw ? cc : 0u);
             const u32 x = (u32)t;
             cc = t >> 32;
             o[5 + 4 * w + 0] = (u8)x;
@@ -306,42 +255,18 @@ template <int AW> __device__ void final_query_wide(const Query* q, const u32* pa
     }
 }
 
-template <int AW> __device__ void final_query(const Query* q, const u32* partials)
-{
-    Mag<AW> acc = mzero<AW>();
-    for (u32 k = threadIdx.x; k < q->nitems; k += 64) {
-        const u32* p = partials + (usize)(q->item0 + k) * kMaxAccWords;
-        Mag<AW> o;
-#pragma unroll
-        for (int w = 0; w < AW; w++) o.w[w] = p[w];
-        add_to<AW>(acc, acc, o);
-    }
-    wave_reduce<AW>(acc);
-    if (threadIdx.x == 0) {
-        write_sum_image<AW>(q->image, acc, q->outP & 0xffu, q->outS & 0xffu, 0u);
-        *q->count = (int64_t)q->rows;
-    }
-}
-
-__global__ void __launch_bounds__(64) k_vm_final(const Header* h, const Query* qs, const u32* partials)
-{
-    const u32 qi = blockIdx.x;
-    if (qi >= h->nqueries) return;
-    const Query* q = qs + qi;
-    switch (q->wclass) {
-    case 0: final_query<4>(q, partials); break;
-    case 1: final_query<6>(q, partials); break;
-    case 2: final_query<10>(q, partials); break;
-    case 3: final_query<18>(q, partials); break;
-    case 4: final_query<34>(q, partials); break;
-    case 5: final_query_wide<66>(q, partials); break;
-    case 6: final_query_wide<130>(q, partials); break;
-    case 7: final_query_wide<258>(q, partials); break;
-    default: final_query_wide<514>(q, partials); break;
-    }
-}
-
 // ---------------------------------------------------------------- host
+
+// one kernel per register class, one for all wide ones
+constexpr int kNumKernels = kFirstMultiLane + 1;
+constexpr size_t kMaxWorkspace = (size_t)1 << 30;
+constexpr size_t kWideRow = 64 * sizeof(uint32_t);   // bytes of one limb of a wave's 64 values
+
+// words of a program as the kernels read it
+uint32_t program_words(const VmProgram& p)
+{
+    return p.wide.empty() ? 3u * (uint32_t)p.ins.size() : (uint32_t)p.wide.size();
+}
 
 struct Pending {
     std::shared_ptr<const VmProgram> prog;
@@ -375,9 +300,13 @@ struct updec_batch_s {
     int max_queries = 0, max_items = 0, max_prog_words = 0, max_const_words = 0;
     // defaults sized so one 10^7-row query alone makes >= 4 items per CU
     int64_t rows_per_item[kNumClasses] = {8192, 8192, 4096, 2048, 1024, 512, 256, 128, 64};
-    int blocks_per_cu[kNumClasses] = {4, 4, 4, 4, 4, 4, 4, 4, 4};
-    // lanes per value of the multi-lane classes: W / 4 (4 limbs per lane) or W / 8 (8 limbs)
-    int lanes[kNumClasses] = {1, 1, 1, 1, 1, 16, 32, 64, 64};
+    // (a block of the wide classes is one wave)
+    int blocks_per_cu[kNumClasses] = {4, 4, 4, 4, 4, 12, 12, 12, 12};
+    // workspace of the wide kernel, grown by updec_batch_add to what the
+    // largest wide program met so far needs, at most kMaxWorkspace
+    uint8_t* d_work = nullptr;
+    size_t work_bytes = 0;
+    size_t pend_stride = 0;   // bytes per block of the pending queries' largest
     Header* h_hdr = nullptr;
     Query* h_q = nullptr;
     Item* h_items = nullptr;
@@ -391,8 +320,8 @@ struct updec_batch_s {
     uint32_t* d_partials = nullptr;
     hipEvent_t staged = nullptr;  // the last launch's host-to-device copies are done
     bool staged_pending = false;
-    hipStream_t side[kNumClasses] = {};
-    hipEvent_t fork = nullptr, join[kNumClasses] = {};
+    hipStream_t side[kNumKernels] = {};
+    hipEvent_t fork = nullptr, join[kNumKernels] = {};
     hipGraphExec_t graph = nullptr;
     std::vector<Pending> pending;
     // space the pending queries take at launch
@@ -421,61 +350,90 @@ struct updec_batch_s {
         (void)hipFree(d_prog);
         (void)hipFree(d_cst);
         (void)hipFree(d_partials);
+        (void)hipFree(d_work);
     }
 
     void clear_pending()
     {
         pending.clear();
         pend_items = pend_prog_words = pend_const_words = 0;
+        pend_stride = 0;
         pend_programs.clear();
     }
 
-    int grid(int cls, uint32_t nitems) const
+    // blocks of the wide kernel on a full device
+    int wide_grid() const
     {
-        const int g = api_device_cus() * blocks_per_cu[cls];
-        return std::max(1, std::min<int>(g, (int)nitems));
+        int bpc = 1;
+        for (int c = kFirstMultiLane; c < kNumClasses; c++) bpc = std::max(bpc, blocks_per_cu[c]);
+        return api_device_cus() * bpc;
+    }
+
+    // workspace for blocks of `stride` bytes: for every block of a full
+    // device up to kMaxWorkspace, and where that much memory is not free, for
+    // as many as there is (64 at least)
+    int reserve(size_t stride)
+    {
+        const size_t most = std::max(kMaxWorkspace, 64 * stride);
+        size_t want = std::min(most, (size_t)wide_grid() * stride);
+        if (want <= work_bytes) return UPDEC_OK;
+        want = std::min(most, std::max(want, work_bytes + work_bytes / 2));
+        // launches that use the old one are waited for
+        if (d_work) VMCHK(hipFree(d_work));
+        d_work = nullptr;
+        work_bytes = 0;
+        while (hipMalloc(reinterpret_cast<void**>(&d_work), want) != hipSuccess) {
+            (void)hipGetLastError();
+            d_work = nullptr;
+            want /= 2;
+            if (want < 64 * stride) return api_fail(UPDEC_EHIP, "no device memory for the wide kernel's workspace");
+        }
+        work_bytes = want;
+        return UPDEC_OK;
     }
 
     // launch the class kernels (on `s` or on the side streams) and the final kernel
     int launch_kernels(hipStream_t s, bool fork_join, const uint32_t* nitems_per_class)
     {
-        auto launch_class = [&](int c, hipStream_t st) -> int {
-            const int g = nitems_per_class ? grid(c, nitems_per_class[c]) : api_device_cus() * blocks_per_cu[c];
-            switch (c) {
+        // kernel k: class k of the register classes, or all the wide ones
+        auto items_of = [&](int k) {
+            uint32_t n = 0;
+            for (int c = k; c < (k < kFirstMultiLane ? k + 1 : kNumClasses); c++) n += nitems_per_class[c];
+            return n;
+        };
+        auto launch_kernel = [&](int k, hipStream_t st) -> int {
+            int g = k < kFirstMultiLane ? api_device_cus() * blocks_per_cu[k] : wide_grid();
+            if (nitems_per_class) g = std::max(1, std::min<int>(g, (int)items_of(k)));
+            switch (k) {
             case 0: hipLaunchKernelGGL((k_vm_sum<2, kBlock[0]>), dim3(g), dim3(kBlock[0]), 0, st, d_hdr, d_q, d_prog, d_cst, d_items, d_partials); break;
             case 1: hipLaunchKernelGGL((k_vm_sum<4, kBlock[1]>), dim3(g), dim3(kBlock[1]), 0, st, d_hdr, d_q, d_prog, d_cst, d_items, d_partials); break;
             case 2: hipLaunchKernelGGL((k_vm_sum<8, kBlock[2]>), dim3(g), dim3(kBlock[2]), 0, st, d_hdr, d_q, d_prog, d_cst, d_items, d_partials); break;
             case 3: hipLaunchKernelGGL((k_vm_sum<16, kBlock[3]>), dim3(g), dim3(kBlock[3]), 0, st, d_hdr, d_q, d_prog, d_cst, d_items, d_partials); break;
             case 4: hipLaunchKernelGGL((k_vm_sum<32, kBlock[4]>), dim3(g), dim3(kBlock[4]), 0, st, d_hdr, d_q, d_prog, d_cst, d_items, d_partials); break;
-#define UPD_ML(Lx, TPIx, C) hipLaunchKernelGGL((k_vm_sum_ml<Lx, TPIx, kBlock[C]>), dim3(g), dim3(kBlock[C]), 0, st, d_hdr, d_q, d_prog, d_cst, d_items, d_partials)
-            case 5: if (lanes[5] == 8) UPD_ML(8, 8, 5); else UPD_ML(4, 16, 5); break;
-            case 6: if (lanes[6] == 16) UPD_ML(8, 16, 6); else UPD_ML(4, 32, 6); break;
-            case 7: if (lanes[7] == 32) UPD_ML(8, 32, 7); else UPD_ML(4, 64, 7); break;
-            default: UPD_ML(8, 64, 8); break;   // 512 limbs: a whole wave, 8 limbs per lane
-#undef UPD_ML
+            default: hipLaunchKernelGGL(k_vm_sum_wide, dim3(g), dim3(64), 0, st, d_hdr, d_q, d_prog, d_cst, d_items, d_partials); break;
             }
             VMCHK(hipGetLastError());
             return UPDEC_OK;
         };
         if (fork_join) {
             VMCHK(hipEventRecord(fork, s));
-            for (int c = 0; c < kNumClasses; c++) {
-                VMCHK(hipStreamWaitEvent(side[c], fork, 0));
-                int rc = launch_class(c, side[c]);
+            for (int k = 0; k < kNumKernels; k++) {
+                VMCHK(hipStreamWaitEvent(side[k], fork, 0));
+                int rc = launch_kernel(k, side[k]);
                 if (rc) return rc;
-                VMCHK(hipEventRecord(join[c], side[c]));
-                VMCHK(hipStreamWaitEvent(s, join[c], 0));
+                VMCHK(hipEventRecord(join[k], side[k]));
+                VMCHK(hipStreamWaitEvent(s, join[k], 0));
             }
         } else {
-            for (int c = 0; c < kNumClasses; c++) {
-                if (nitems_per_class && nitems_per_class[c] == 0) continue;
-                int rc = launch_class(c, s);
+            for (int k = 0; k < kNumKernels; k++) {
+                if (nitems_per_class && items_of(k) == 0) continue;
+                int rc = launch_kernel(k, s);
                 if (rc) return rc;
             }
         }
         const uint32_t nq = fork_join ? (uint32_t)max_queries : h_hdr->nqueries;
         if (nq) {
-            hipLaunchKernelGGL(k_vm_final, dim3(nq), dim3(64), 0, s, d_hdr, d_q, d_partials);
+            hipLaunchKernelGGL(k_vm_final, dim3(nq), dim3(kFinalThreads), 0, s, d_hdr, d_q, d_partials);
             VMCHK(hipGetLastError());
         }
         return UPDEC_OK;
@@ -536,7 +494,7 @@ int updec_batch_create(int32_t max_queries, int32_t max_items, updec_batch_t* ou
     std::unique_ptr<updec_batch_s> b(new updec_batch_s());
     b->max_queries = max_queries;
     b->max_items = max_items;
-    b->max_prog_words = max_queries * 3 * 64;
+    b->max_prog_words = max_queries * (3 * 64 + (int)wide::kHead);
     b->max_const_words = max_queries * 8 * (512 + 1);
     int rc;
     if ((rc = host_alloc(&b->h_hdr, 1)) || (rc = host_alloc(&b->h_q, max_queries)) || (rc = host_alloc(&b->h_items, max_items)) ||
@@ -548,7 +506,7 @@ int updec_batch_create(int32_t max_queries, int32_t max_items, updec_batch_t* ou
     memset(b->h_hdr, 0, sizeof(Header));
     VMCHK(hipEventCreateWithFlags(&b->staged, hipEventDisableTiming));
     VMCHK(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
-    for (int c = 0; c < kNumClasses; c++) {
+    for (int c = 0; c < kNumKernels; c++) {
         VMCHK(hipStreamCreateWithFlags(&b->side[c], hipStreamNonBlocking));
         VMCHK(hipEventCreateWithFlags(&b->join[c], hipEventDisableTiming));
     }
@@ -575,18 +533,13 @@ int updec_batch_tuning(updec_batch_t b, int32_t width_class, int64_t rows_per_it
 int updec_batch_lanes(updec_batch_t b, int32_t width_class, int32_t lanes)
 {
     if (!b || width_class < kFirstMultiLane || width_class >= kNumClasses)
-        return api_fail(UPDEC_EINVAL, "lanes per value apply to the multi-lane classes (W = 64 .. 512)");
+        return api_fail(UPDEC_EINVAL, "lanes per value apply to the wide classes (W = 64 .. 512)");
     const int W = kClassW[width_class];
     if ((lanes != W / 4 && lanes != W / 8) || lanes > 64)
         return api_fail(UPDEC_EINVAL, "lanes per value must be W / 4 or W / 8, at most 64");
     std::lock_guard<std::mutex> g(b->mu);
     if (!b->pending.empty()) return api_fail(UPDEC_EINVAL, "tuning changes while queries are staged");
-    b->lanes[width_class] = lanes;
-    if (b->graph) {
-        (void)hipGraphExecDestroy(b->graph);
-        b->graph = nullptr;
-    }
-    return UPDEC_OK;
+    return UPDEC_OK;   // a value lies in one lane's memory whatever is asked
 }
 
 int updec_batch_add(updec_batch_t b, updec_vm_t v, const uint8_t* const* d_cols, int64_t rows, uint8_t* d_image,
@@ -603,13 +556,19 @@ int updec_batch_add(updec_batch_t b, updec_vm_t v, const uint8_t* const* d_cols,
     // blocks): four items per block keep the load balanced while the
     // per-item work (fetch, block reduction, partial write) stays small next
     // to the item's rows
+    // (for the wide classes, whose items are one wave's, a small query is
+    // spread over as many waves as its share of the items allows)
+    if (!pr.wide.empty()) {
+        const int64_t share = std::max<int64_t>(1, std::min<int64_t>(b->max_items / b->max_queries, 1024));
+        ch = std::min(ch, std::max<int64_t>(64, (rows + share * 64 - 1) / (share * 64) * 64));
+    }
     const int64_t slots = 4 * (int64_t)api_device_cus() * b->blocks_per_cu[pr.wclass];
     const int64_t big = (rows + slots - 1) / slots;
     if (big > ch) ch = (big + 63) / 64 * 64;
     if ((rows + ch - 1) / ch > b->max_items) ch = ((rows + b->max_items - 1) / b->max_items + 63) / 64 * 64;
     const uint32_t items = (uint32_t)std::max<int64_t>(1, (rows + ch - 1) / ch);
     const bool new_prog = b->pend_programs.find(&pr) == b->pend_programs.end();
-    const uint32_t pw = new_prog ? 3u * (uint32_t)pr.ins.size() : 0u, cw = new_prog ? (uint32_t)pr.consts.size() : 0u;
+    const uint32_t pw = new_prog ? program_words(pr) : 0u, cw = new_prog ? (uint32_t)pr.consts.size() : 0u;
     if ((int)b->pending.size() >= b->max_queries || b->pend_items + items > (uint32_t)b->max_items ||
         b->pend_prog_words + pw > (uint32_t)b->max_prog_words || b->pend_const_words + cw > (uint32_t)b->max_const_words) {
         if (b->pending.empty()) return api_fail(UPDEC_EINVAL, "query does not fit an empty batch");
@@ -626,6 +585,11 @@ int updec_batch_add(updec_batch_t b, updec_vm_t v, const uint8_t* const* d_cols,
     p.chunk = ch;
     p.image = d_image;
     p.count = d_count;
+    if (!pr.wide.empty()) {
+        const size_t stride = (size_t)pr.wide_rows * kWideRow;
+        if (int rc = b->reserve(std::max(stride, b->pend_stride))) return rc;
+        b->pend_stride = std::max(stride, b->pend_stride);
+    }
     b->pending.push_back(p);
     b->pend_items += items;
     b->pend_prog_words += pw;
@@ -675,6 +639,9 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
     Header& H = *b->h_hdr;
     memset(&H, 0, sizeof H);
     H.nqueries = (uint32_t)b->pending.size();
+    H.workspace = b->d_work;
+    H.stride = b->pend_stride;
+    H.wide_blocks = b->pend_stride ? (uint32_t)std::min<size_t>(b->work_bytes / b->pend_stride, (size_t)INT32_MAX) : 0u;
     for (int c = 0; c < kNumClasses; c++) {
         H.class_item0[c] = first[c];
         H.class_nitems[c] = nitems[c];
@@ -684,12 +651,13 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
         const VmProgram& pr = *p.prog;
         auto it = placed.find(&pr);
         if (it == placed.end()) {
-            const uint32_t pw = 3u * (uint32_t)pr.ins.size(), cw = (uint32_t)pr.consts.size();
+            const uint32_t pw = program_words(pr), cw = (uint32_t)pr.consts.size();
             if (prog_words + pw > (uint32_t)b->max_prog_words || const_words + cw > (uint32_t)b->max_const_words) {
                 b->clear_pending();
                 return api_fail(UPDEC_EINVAL, "batch programs exceed the staging space");
             }
-            for (size_t k = 0; k < pr.ins.size(); k++) {
+            if (!pr.wide.empty()) memcpy(b->h_prog + prog_words, pr.wide.data(), 4u * pw);
+            for (size_t k = 0; pr.wide.empty() && k < pr.ins.size(); k++) {
                 const Ins& I = pr.ins[k];
                 uint32_t* w = b->h_prog + prog_words + 3 * k;
                 w[0] = (uint32_t)I.op | ((uint32_t)I.dst << 8) | ((uint32_t)I.arg << 16);
@@ -697,6 +665,13 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
                 w[2] = (uint32_t)I.b.kind | ((uint32_t)I.b.idx << 8) | ((uint32_t)I.b.shift << 16);
             }
             if (cw) memcpy(b->h_cst + const_words, pr.consts.data(), 4u * cw);
+            if (!pr.wide.empty())
+                // a constant's sign word also tells its limbs
+                for (uint32_t* k = b->h_cst + const_words; k < b->h_cst + const_words + cw; k += pr.W + 1) {
+                    uint32_t n = (uint32_t)pr.W;
+                    while (n > 0 && k[n] == 0u) n--;
+                    *k = (*k & 1u) | (n << 8);
+                }
             it = placed.emplace(&pr, std::make_pair(prog_words / 3u, const_words)).first;
             prog_words += pw;
             const_words += cw;
