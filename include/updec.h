@@ -246,8 +246,9 @@ int updec_agg_compile(const updec_agg_desc* desc, updec_agg_t* out);
 int updec_agg_run(updec_agg_t a, const uint8_t* const* d_cols, const int32_t* d_filter, const uint8_t* d_key0,
                   const uint8_t* d_key1, int64_t rows, uint8_t* d_images, int64_t* d_counts, int32_t max_groups,
                   int32_t* ngroups_out, uint16_t* keys_out, updec_stream_t stream);
-/* device time of the last run's main aggregation kernel, in milliseconds
- * (HIP events on the run's stream; synchronizes) */
+/* device time of the last run's main aggregation kernel, in milliseconds:
+ * from its start to the start of the kernel after it, by the device's clock
+ * (synchronizes) */
 int updec_agg_last_kernel_ms(updec_agg_t a, float* ms);
 /* generated source for a given group count of the two-pass form, or of the
  * one-pass form with ngroups = 0 (no device needed) */

@@ -33,6 +33,16 @@ typedef __SIZE_TYPE__ usize;
 template <int W> struct Mag { u32 w[W]; };
 template <int W> struct Dec { Mag<W> m; u32 neg; };
 
+// the device's constant-rate clock
+UPD_DEV u64 device_clock()
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_readsteadycounter();
+#else
+    return 0;
+#endif
+}
+
 // ---------------------------------------------------------------- constants
 
 // Exact 10^n as 32-bit words, built at compile time (n <= 460).

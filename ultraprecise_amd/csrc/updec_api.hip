@@ -603,6 +603,8 @@ struct updec_agg_s {
     std::map<int, GenMod> by_ngroups;
     u32* d_bitmap = nullptr;
     u8* d_lut = nullptr;
+    static constexpr size_t kClockBytes = 256;
+    static constexpr size_t kMetaClock = 4 + 256;  // word of h_meta
     u32* d_partials = nullptr;
     size_t partial_words = 0;
     // one-pass grouped form
@@ -623,17 +625,33 @@ struct updec_agg_s {
     // [4..] keys
     u32* h_meta = nullptr;
     u32* h_meta_dev = nullptr;  // its device address
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    // clock readings of the last run, which its kernels write (start of the
+    // main kernel, start of the final one): a one-pass run's follow h_meta's
+    // keys, a two-pass run's head the allocation of the partials, which
+    // needs no pinned memory otherwise
+    u64* d_clk = nullptr;
+    const u64* clk_host = nullptr;  // where the last run's can be read; null: copy from d_clk
     bool timed = false;
+    int reserve_partials(size_t words)
+    {
+        if (words <= partial_words) return UPDEC_OK;
+        timed = false;
+        if (d_clk) HIPCHK(hipFree(d_clk));
+        d_clk = nullptr;
+        d_partials = nullptr;
+        partial_words = 0;
+        HIPCHK(hipMalloc((void**)&d_clk, kClockBytes + words * sizeof(u32)));
+        d_partials = reinterpret_cast<u32*>(d_clk + kClockBytes / sizeof(u64));
+        partial_words = words;
+        return UPDEC_OK;
+    }
     ~updec_agg_s()
     {
         if (d_bitmap) (void)hipFree(d_bitmap);
         if (d_lut) (void)hipFree(d_lut);
-        if (d_partials) (void)hipFree(d_partials);
+        if (d_clk) (void)hipFree(d_clk);
         if (d_meta) (void)hipFree(d_meta);
         if (h_meta) (void)hipHostFree(h_meta);
-        if (ev0) (void)hipEventDestroy(ev0);
-        if (ev1) (void)hipEventDestroy(ev1);
     }
 };
 
@@ -1229,18 +1247,13 @@ static int agg_run_onepass(updec_agg_t a, const uint8_t* const* d_cols, const in
     const int T = a->op_block;
     const int64_t grid = agg_grid(fmain, rows, T, agg_rows_per_step(a->spec, a->types, GenOptions()));
     const size_t need = (size_t)grid * (size_t)agg_onepass_record_words(a->spec);
-    if (need > a->partial_words) {
-        if (a->d_partials) HIPCHK(hipFree(a->d_partials));
-        a->d_partials = nullptr;
-        HIPCHK(hipMalloc((void**)&a->d_partials, need * sizeof(u32)));
-        a->partial_words = need;
-    }
+    if (int rc = a->reserve_partials(need)) return rc;
     if (!a->d_meta) {
         HIPCHK(hipMalloc((void**)&a->d_meta, 2 * kAggOnepassStatWords * sizeof(u32)));
         a->stat_dirty = true;
     }
     if (!a->h_meta) {
-        HIPCHK(hipHostMalloc((void**)&a->h_meta, (4 + 256) * sizeof(u32), hipHostMallocMapped | hipHostMallocCoherent));
+        HIPCHK(hipHostMalloc((void**)&a->h_meta, updec_agg_s::kMetaClock * sizeof(u32) + 2 * sizeof(u64), hipHostMallocMapped | hipHostMallocCoherent));
         HIPCHK(hipHostGetDevicePointer((void**)&a->h_meta_dev, a->h_meta, 0));
     }
     if (a->stat_dirty) HIPCHK(hipMemsetAsync(a->d_meta, 0, 2 * kAggOnepassStatWords * sizeof(u32), st));
@@ -1251,31 +1264,23 @@ static int agg_run_onepass(updec_agg_t a, const uint8_t* const* d_cols, const in
     AggArgs args;
     fill_args(a, &args, d_cols, d_filter, d_key0, d_key1, rows);
     u32* ovf = stat;
-    if (!a->ev0) {
-        HIPCHK(hipEventCreate(&a->ev0));
-        HIPCHK(hipEventCreate(&a->ev1));
-    }
-    // events recorded around the launch (events attached to the dispatch
-    // with hipExtModuleLaunchKernel cost about 16 us more host time per
-    // launch); the span also takes in the few microseconds between the first
-    // marker and the dispatch
-    void* pm[] = {&args, &ovf};
-    HIPCHK(hipEventRecord(a->ev0, st));
+    u64* clk = reinterpret_cast<u64*>(a->h_meta_dev + updec_agg_s::kMetaClock);
+    void* pm[] = {&args, &ovf, &clk};
     HIPCHK(hipModuleLaunchKernel(fmain, (uint32_t)grid, 1, 1, T, 1, 1, 0, st, pm, nullptr));
-    HIPCHK(hipEventRecord(a->ev1, st));
-    a->timed = true;
     const u32* rec = a->d_partials;
     u32 nb = (u32)grid, maxg = (u32)max_groups;
     uint8_t* img = d_images;
     uint64_t* cnt = reinterpret_cast<uint64_t*>(d_counts);
     u32* meta = a->h_meta_dev;
     uint8_t* avgs = a->spec.avg_mask ? d_images + (size_t)max_groups * a->spec.plans.size() * 133 : nullptr;
-    void* pf[] = {&rec, &nb, &stat, &next, &maxg, &img, &cnt, &meta, &avgs};
+    void* pf[] = {&rec, &nb, &stat, &next, &maxg, &img, &cnt, &meta, &avgs, &clk};
     const int NP = (int)a->spec.plans.size();
     HIPCHK(hipModuleLaunchKernel(ffin, (unsigned)(max_groups * (NP + 1)), 1, 1, kAggFinalThreads, 1, 1, 0, st, pf, nullptr));
     a->stat_dirty = false;
     a->stat_phase = 1 - a->stat_phase;
     HIPCHK(hipStreamSynchronize(st));
+    a->timed = true;
+    a->clk_host = reinterpret_cast<const u64*>(a->h_meta + updec_agg_s::kMetaClock);
     if (a->h_meta[2]) {
         *overflowed = true;
         return UPDEC_OK;
@@ -1350,16 +1355,12 @@ static int agg_run_twopass(updec_agg_t a, const IterArgs* iter, const uint8_t* c
     GenOptions go;
     go.blocks = iter != nullptr;
     const int64_t grid = agg_grid(fmain, rows, T, agg_rows_per_step(a->spec, a->types, go));
-    if ((size_t)grid * PW > a->partial_words) {
-        if (a->d_partials) HIPCHK(hipFree(a->d_partials));
-        a->d_partials = nullptr;
-        HIPCHK(hipMalloc((void**)&a->d_partials, (size_t)grid * PW * sizeof(u32)));
-        a->partial_words = (size_t)grid * PW;
-    }
+    if (int rc = a->reserve_partials((size_t)grid * PW)) return rc;
     if (int krc = a->consts.upload(st)) return krc;
     AggArgs args;
     IterArgs iargs;
-    void* pm[1];
+    u64* clk = a->d_clk;
+    void* pm[2] = {nullptr, &clk};
     if (iter) {
         iargs = *iter;
         iargs.fcol = d_filter;
@@ -1373,20 +1374,15 @@ static int agg_run_twopass(updec_agg_t a, const IterArgs* iter, const uint8_t* c
         fill_args(a, &args, d_cols, d_filter, d_key0, d_key1, rows);
         pm[0] = &args;
     }
-    if (!a->ev0) {
-        HIPCHK(hipEventCreate(&a->ev0));
-        HIPCHK(hipEventCreate(&a->ev1));
-    }
-    HIPCHK(hipEventRecord(a->ev0, st));
     HIPCHK(hipModuleLaunchKernel(fmain, (uint32_t)grid, 1, 1, T, 1, 1, 0, st, pm, nullptr));
-    HIPCHK(hipEventRecord(a->ev1, st));
-    a->timed = true;
     const u32* cp = a->d_partials;
     u32 nb = (u32)grid;
     uint8_t* img = d_images;
     uint64_t* cnt = reinterpret_cast<uint64_t*>(d_counts);
-    void* pf[] = {&cp, &nb, &img, &cnt};
+    void* pf[] = {&cp, &nb, &img, &cnt, &clk};
     HIPCHK(hipModuleLaunchKernel(ffin, (unsigned)(NP * ngroups + ngroups), 1, 1, 256, 1, 1, 0, st, pf, nullptr));
+    a->timed = true;
+    a->clk_host = nullptr;
     return launch_avgs(a, d_images, d_counts, ngroups, max_groups, st);
 }
 
@@ -1448,8 +1444,23 @@ int updec_agg_run_iter(updec_agg_t a, const updec_column_iter* cols, int64_t row
 int updec_agg_last_kernel_ms(updec_agg_t a, float* ms)
 {
     if (!a || !ms || !a->timed) return fail(UPDEC_EINVAL, "no timed run");
-    HIPCHK(hipEventSynchronize(a->ev1));
-    HIPCHK(hipEventElapsedTime(ms, a->ev0, a->ev1));
+    u64 clk[2];
+    if (a->clk_host) {  // the run has been waited for
+        clk[0] = a->clk_host[0];
+        clk[1] = a->clk_host[1];
+    } else {
+        HIPCHK(hipDeviceSynchronize());  // the run's stream may be a non-blocking one
+        HIPCHK(hipMemcpy(clk, a->d_clk, sizeof(clk), hipMemcpyDeviceToHost));
+    }
+    static std::atomic<int> khz{0};
+    if (!khz.load()) {
+        int dev = 0, v = 0;
+        HIPCHK(hipGetDevice(&dev));
+        HIPCHK(hipDeviceGetAttribute(&v, hipDeviceAttributeWallClockRate, dev));
+        if (v <= 0) return fail(UPDEC_EHIP, "the device reports no clock rate");
+        khz.store(v);
+    }
+    *ms = (float)((double)(i64)(clk[1] - clk[0]) / khz.load());
     return UPDEC_OK;
 }
 
