@@ -556,12 +556,6 @@ int updec_batch_add(updec_batch_t b, updec_vm_t v, const uint8_t* const* d_cols,
     // blocks): four items per block keep the load balanced while the
     // per-item work (fetch, block reduction, partial write) stays small next
     // to the item's rows
-    // (for the wide classes, whose items are one wave's, a small query is
-    // spread over as many waves as its share of the items allows)
-    if (!pr.wide.empty()) {
-        const int64_t share = std::max<int64_t>(1, std::min<int64_t>(b->max_items / b->max_queries, 1024));
-        ch = std::min(ch, std::max<int64_t>(64, (rows + share * 64 - 1) / (share * 64) * 64));
-    }
     const int64_t slots = 4 * (int64_t)api_device_cus() * b->blocks_per_cu[pr.wclass];
     const int64_t big = (rows + slots - 1) / slots;
     if (big > ch) ch = (big + 63) / 64 * 64;
@@ -620,8 +614,22 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
     }
     // items per class, in class order; programs and constants deduplicated
     uint32_t nitems[kNumClasses] = {};
-    for (const Pending& p : b->pending) {
+    // The rows per item of updec_batch_add suit queries that fill the device;
+    // one of 50,000 rows had 7 to 49 of its blocks.  Where a kernel's rows
+    // would leave it with fewer than two items for each resident block, its
+    // queries are cut finer, down to one row a thread, as far as the items
+    // that the batch has to spare go (dealt out evenly): one query of 50,000
+    // rows 714 -> 151 us at 16 limbs, 274 -> 127 at 2; 1.2 M rows at 16 limbs
+    // 783 -> 550.
+    const int64_t spare = (b->max_items - (int64_t)b->pend_items) / (int64_t)b->pending.size();
+    int64_t rows_of[kNumKernels] = {};
+    for (const Pending& p : b->pending) rows_of[std::min(p.prog->wclass, kFirstMultiLane)] += p.rows;
+    for (Pending& p : b->pending) {
         const int c = p.prog->wclass;
+        const int64_t T = p.prog->wide.empty() ? kBlock[c] : 64;
+        const int64_t most = std::max<int64_t>(1, (p.rows + p.chunk - 1) / p.chunk) + spare;
+        const int64_t even = rows_of[std::min(c, kFirstMultiLane)] / (2 * (int64_t)api_device_cus() * b->blocks_per_cu[c]);
+        p.chunk = std::min(p.chunk, std::max(T, (std::max(even, (p.rows + most - 1) / most) + T - 1) / T * T));
         nitems[c] += (uint32_t)std::max<int64_t>(1, (p.rows + p.chunk - 1) / p.chunk);
     }
     uint32_t total = 0, first[kNumClasses];
