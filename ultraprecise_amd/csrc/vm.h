@@ -94,6 +94,8 @@ struct Query {
     uint32_t faithful;        // DivOrMod path quirks
     uint32_t wclass;          // index into kClassW
     uint32_t item0, nitems;   // this query's work items (contiguous)
+    uint32_t done;            // blocks of the final kernel that have ended
+    uint32_t pad;
     uint8_t* image;           // 133-byte nullable_type<Decimal> of SUM
     int64_t* count;           // COUNT(*)
 };

@@ -191,22 +191,36 @@ __global__ void __launch_bounds__(64, 3)
     }
 }
 
-// SUM image and COUNT of every query: one block each.  Lanes take the words
-// of the items' partials (consecutive words of an item, as many items at once
-// as fit a wave), waves take items in turn; the words are added without
-// carries as 64-bit sums, then one carry pass, and the image gets the low 32
-// limbs of the magnitude.
+// SUM image and COUNT of every query.  Lanes take the words of the items'
+// partials (consecutive words of an item, as many items at once as fit a
+// wave), waves take items in turn; the words are added without carries as
+// 64-bit sums, then one carry pass, and the image gets the low 32 limbs of
+// the magnitude.  A query of many items has several blocks, each for a
+// contiguous part of them; the one that ends last adds their sums, which the
+// others left in their first two items' places.
 //
 // What bounds it: latency of the partials' loads.  With one wave per query,
 // walking the items one after the other, 7,800 partials of a 256-limb query
-// took 6 ms, now 0.1.
+// took 6 ms; the 12,000 partials of such a query at 9 M rows took one block of
+// 16 waves 1.6 ms, several 0.19.  Up to
+// 1,000 items a query stays with one block: two that share 391 items take 7 us
+// longer for handing over.
 constexpr int kFinalThreads = 1024, kFinalAhead = 4;
-__global__ void __launch_bounds__(kFinalThreads) k_vm_final(const Header* h, const Query* qs, const u32* partials)
+constexpr u32 kFinalSlices = 16, kSliceItems = 512;   // blocks a query at most, items a block at least
+constexpr u32 kFinalBlocks = 2048;                    // of all queries, where one a query are fewer
+UPD_DEV u64* slice_sums(u32* partials, const Query* q, u32 y, u32 n)
+{
+    return reinterpret_cast<u64*>(partials + (usize)(q->item0 + (u32)((u64)q->nitems * y / n)) * kMaxAccWords);
+}
+__global__ void __launch_bounds__(kFinalThreads) k_vm_final(const Header* h, Query* qs, u32* partials)
 {
     __shared__ u64 cs[kMaxAccWords];
-    const u32 qi = blockIdx.x, tid = threadIdx.x;
+    __shared__ u32 s_last;
+    const u32 qi = blockIdx.x, tid = threadIdx.x, y = blockIdx.y;
     if (qi >= h->nqueries) return;
-    const Query* q = qs + qi;
+    Query* q = qs + qi;
+    const u32 parts = q->nitems / kSliceItems, n = parts < 1u ? 1u : parts < gridDim.y ? parts : gridDim.y;
+    if (y >= n) return;
     const u32 aw = ((u32)kClassW[0] << q->wclass) + 2u;
     for (u32 w = tid; w < aw; w += kFinalThreads) cs[w] = 0;
     __syncthreads();
@@ -214,17 +228,34 @@ __global__ void __launch_bounds__(kFinalThreads) k_vm_final(const Header* h, con
     u32 wide = 4;
     while (wide < aw && wide < 64u) wide <<= 1;
     const u32 rows = kFinalThreads / wide, row = tid / wide;
+    const u32 k0 = (u32)((u64)q->nitems * y / n), k1 = (u32)((u64)q->nitems * (y + 1u) / n);
     const u32* base = partials + (usize)q->item0 * kMaxAccWords;
     for (u32 w = tid % wide; w < aw; w += wide) {
         u64 s = 0;
-        for (u32 k = row; k < q->nitems; k += rows * kFinalAhead) {
+        for (u32 k = k0 + row; k < k1; k += rows * kFinalAhead) {
 #pragma unroll
             for (u32 t = 0; t < (u32)kFinalAhead; t++)
-                if (k + t * rows < q->nitems) s += base[(usize)(k + t * rows) * kMaxAccWords + w];
+                if (k + t * rows < k1) s += base[(usize)(k + t * rows) * kMaxAccWords + w];
         }
         if (s) atomicAdd(reinterpret_cast<unsigned long long*>(&cs[w]), (unsigned long long)s);
     }
     __syncthreads();
+    if (n > 1u) {
+        u64* mine = slice_sums(partials, q, y, n);
+        for (u32 w = tid; w < aw; w += kFinalThreads) __hip_atomic_store(mine + w, cs[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __threadfence();
+        __syncthreads();
+        if (tid == 0) s_last = __hip_atomic_fetch_add(&q->done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u == n ? 1u : 0u;
+        __syncthreads();
+        if (!s_last) return;
+        __threadfence();
+        for (u32 w = tid; w < aw; w += kFinalThreads) {
+            u64 s = 0;
+            for (u32 k = 0; k < n; k++) s += __hip_atomic_load(slice_sums(partials, q, k, n) + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            cs[w] = s;
+        }
+        __syncthreads();
+    }
     if (tid == 0) {
         u64 c = 0;
         for (u32 w = 0; w < aw; w++) {
@@ -458,7 +489,8 @@ struct updec_batch_s {
         }
         const uint32_t nq = fork_join ? (uint32_t)max_queries : h_hdr->nqueries;
         if (nq) {
-            hipLaunchKernelGGL(k_vm_final, dim3(nq), dim3(kFinalThreads), 0, s, d_hdr, d_q, d_partials);
+            const u32 slices = std::min(kFinalSlices, std::max(1u, kFinalBlocks / nq));
+            hipLaunchKernelGGL(k_vm_final, dim3(nq, slices), dim3(kFinalThreads), 0, s, d_hdr, d_q, d_partials);
             VMCHK(hipGetLastError());
         }
         return UPDEC_OK;
