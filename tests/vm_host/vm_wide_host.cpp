@@ -24,21 +24,21 @@ using namespace updec_vm;
 
 // out: the 1024-limb two's complement sum of the materialized rows
 extern "C" int vmw_sum(const char* text, const char** names, const int* P, const int* S, int ncols,
-                       const uint8_t* const* data, int64_t rows, uint32_t* out, int* width, char* err, int cap)
+                       const uint8_t* const* data, int64_t rows, uint32_t* out, int* width, char* err, int cap, int mode)
 {
     std::vector<std::string> nm;
     std::vector<ColumnType> ty(ncols);
     for (int i = 0; i < ncols; i++) { nm.push_back(names[i]); ty[i].P = P[i]; ty[i].S = S[i]; ty[i].bits = 0; }
     Plan plan;
     std::string e;
-    if (!plan_expression(text, nm, ty, 2, &plan, &e)) { snprintf(err, cap, "%s", e.c_str()); return 1; }
+    if (!plan_expression(text, nm, ty, mode, &plan, &e)) { snprintf(err, cap, "%s", e.c_str()); return 1; }
     VmProgram pr;
     if (!build_vm_program(plan, ty, &pr, &e)) { snprintf(err, cap, "%s", e.c_str()); return 2; }
     *width = pr.W;
     if (pr.wide.empty()) { snprintf(err, cap, "no wide form"); return 3; }
     Query Q{};
     for (int c = 0; c < ncols; c++) { Q.col[c] = data[c]; Q.colbytes[c] = compact_bytes(P[c]); }
-    Q.rows = rows; Q.nins = pr.ins.size(); Q.outB = pr.outB;
+    Q.rows = rows; Q.nins = pr.ins.size(); Q.outB = pr.outB; Q.faithful = pr.faithful;
     std::vector<uint32_t> cst = pr.consts;
     for (size_t k = 0; k + pr.W < cst.size(); k += pr.W + 1) {
         uint32_t n = 0;

@@ -2806,7 +2806,14 @@ bool build_vm_program(const Plan& p, const std::vector<ColumnType>& cols, VmProg
         *err = "expression needs more interpreter registers than its width class holds";
         return false;
     }
-    if (updec_vm::runs_wide(prog.wclass, prog.faithful) && !build_wide_program(&prog, cols, err)) return false;
+    int divisions = 0;
+    for (const updec_vm::Ins& i : I) divisions += i.op == updec_vm::OP_DIV;
+    bool wraps = false;
+    for (const PNode& x : p.n) wraps = wraps || (faithful && x.ubits > 1024);
+    if (updec_vm::runs_wide(prog.wclass, divisions, wraps) && !build_wide_program(&prog, cols, err)) {
+        if (prog.wclass >= updec_vm::kFirstMultiLane) return false;
+        err->clear();
+    }
     *out = std::move(prog);
     return true;
 }

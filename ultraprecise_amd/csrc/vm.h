@@ -60,8 +60,25 @@ struct Ins {
     Operand a, b;
 };
 
-// Programs of these classes run on the kernel of vm_wide.h
-constexpr bool runs_wide(int wclass, bool faithful) { return wclass >= kFirstMultiLane && !faithful; }
+// Which programs run on the kernel of vm_wide.h: all that the register kernels
+// have no class for, and those of 16 limbs with three divisions or more and of
+// 32 limbs with two.  The register kernels divide at the class width, a lane's
+// whole window in registers, that one at the limbs the wave has; but its values
+// go through memory, which sums, products and loads of long columns feel.  One
+// query, us, register kernel / vm_wide.h: 1.2 M rows of 16 limbs with 5
+// divisions 1217 / 472, 3 divisions 746 / 407, 2 457 / 339 (700 rows 43 / 46,
+// 50,000 rows 65 / 70), 1 300 / 281 (34 / 37, 54 / 63); of 32 limbs with 5
+// divisions 1734 / 549, 2 936 / 481 (76 / 60, 100 / 88), 1 502 / 633; of 8
+// limbs with 4 divisions 383 / 445.
+// A faithful program only where none of its values can wrap at 32 limbs.
+constexpr int kFirstWide = 3, kWideLimbs = 48;
+constexpr bool runs_wide(int wclass, int divisions, bool wraps)
+{
+    return wclass >= kFirstMultiLane || (wclass >= kFirstWide && divisions * kClassW[wclass] >= kWideLimbs && !wraps);
+}
+// the class under which a program's items are listed in a batch: those of
+// vm_wide.h's kernel lie together, behind the ones of the register kernels
+constexpr int item_class(int wclass, bool wide) { return wide && wclass < kFirstMultiLane ? kFirstMultiLane : wclass; }
 
 // The form of a program that vm_wide.h evaluates (planner.cpp,
 // build_wide_program): a header of kHead words, then kIns words an

@@ -613,7 +613,7 @@ int updec_batch_add(updec_batch_t b, updec_vm_t v, const uint8_t* const* d_cols,
     // blocks): four items per block keep the load balanced while the
     // per-item work (fetch, block reduction, partial write) stays small next
     // to the item's rows
-    const int64_t slots = 4 * (int64_t)api_device_cus() * b->blocks_per_cu[pr.wclass];
+    const int64_t slots = 4 * (int64_t)api_device_cus() * b->blocks_per_cu[item_class(pr.wclass, !pr.wide.empty())];
     const int64_t big = (rows + slots - 1) / slots;
     if (big > ch) ch = (big + 63) / 64 * 64;
     if ((rows + ch - 1) / ch > b->max_items) ch = ((rows + b->max_items - 1) / b->max_items + 63) / 64 * 64;
@@ -680,9 +680,9 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
     // 783 -> 550.
     const int64_t spare = (b->max_items - (int64_t)b->pend_items) / (int64_t)b->pending.size();
     int64_t rows_of[kNumKernels] = {};
-    for (const Pending& p : b->pending) rows_of[std::min(p.prog->wclass, kFirstMultiLane)] += p.rows;
+    for (const Pending& p : b->pending) rows_of[std::min(item_class(p.prog->wclass, !p.prog->wide.empty()), kFirstMultiLane)] += p.rows;
     for (Pending& p : b->pending) {
-        const int c = p.prog->wclass;
+        const int c = item_class(p.prog->wclass, !p.prog->wide.empty());
         const int64_t T = p.prog->wide.empty() ? kBlock[c] : 64;
         const int64_t most = std::max<int64_t>(1, (p.rows + p.chunk - 1) / p.chunk) + spare;
         const int64_t even = rows_of[std::min(c, kFirstMultiLane)] / (2 * (int64_t)api_device_cus() * b->blocks_per_cu[c]);
@@ -759,7 +759,7 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
         Q.wclass = (uint32_t)pr.wclass;
         Q.image = p.image;
         Q.count = p.count;
-        const int c = pr.wclass;
+        const int c = item_class(pr.wclass, !pr.wide.empty());
         const int64_t ch = p.chunk;
         const uint32_t n = (uint32_t)std::max<int64_t>(1, (p.rows + ch - 1) / ch);
         Q.item0 = fill[c];

@@ -1,5 +1,6 @@
-// vm_wide.h -- the interpreter's evaluation of wide programs (vm.h, classes
-// of 64 limbs and more): one lane per row, values in memory.
+// vm_wide.h -- the interpreter's evaluation of wide programs and of those
+// that spend their time in divisions (vm.h, runs_wide): one lane per row,
+// values in memory.
 //
 // A program's register width is the worst case of its widest intermediate;
 // the values themselves are mostly far shorter (a quotient has its scale's
@@ -350,8 +351,9 @@ UPD_DEV u32 digit3by2(u32 u2, u32 u1, u32 u0, u32 d1, u32 d0, u32 v, u64& r, u32
 // limbs of the equally shifted X are taken in from the top, one quotient
 // digit each.  X lies in q's rows: digit j is written when only limbs below
 // j are still to be read.  bl: the lane's bit length of B (not 0).  Returns
-// the limbs of q; rnd = 1 where twice the remainder is at least B.
-template <int NB> UPD_DEV u32 div_reg(const Dst& q, const Src& X, const Src& B, u32 bl, u32& rnd)
+// the limbs of q; rnd = 1 where twice the remainder is at least B; rtop: the
+// shifted remainder's top limb.
+template <int NB> UPD_DEV u32 div_reg(const Dst& q, const Src& X, const Src& B, u32 bl, u32& rnd, u32& rtop)
 {
     const u32 k = 32u * NB - bl, bs = k & 31u;
     const i32 ws = (i32)(k >> 5);
@@ -419,6 +421,7 @@ template <int NB> UPD_DEV u32 div_reg(const Dst& q, const Src& X, const Src& B, 
     Mag<NB> T;
     sub_to<NB>(T, V, win);
     rnd = ge(win, T) ? 1u : 0u;
+    rtop = win.w[NB - 1];
     return wave_max(top);
 }
 
@@ -499,10 +502,55 @@ UPD_DEV u32 div_mem(const Dst& q, const Dst& U, u32 nx, const Src& B, u32 bl, co
     return wave_max(top);
 }
 
-// q = round-half-up(|a| 10^S / |b|), x / 0 = |x| (ddiv's rules, extended
-// mode); q has room for the scaled dividend, U and V as div_mem says; returns
-// the limbs
-UPD_DEV u32 div(const Dst& q, const Src& a, const Src& b, u32 S, const Dst& U, const Dst& V)
+// the lane's bit length of s, from the top
+UPD_DEV u32 bits_of(const Src& s)
+{
+    u32 bl = 0;
+    for (u32 i = s.n; i-- > 0u;) {
+        const u32 x = s.at(i);
+        bl = !bl && x ? 32u * i + 32u - (u32)__builtin_clz(x) : bl;
+        if (!any_lane(bl == 0u)) break;
+    }
+    return bl;
+}
+
+// Where ddiv's faithful rules differ from the exact quotient, by lane:
+// q64 replaces it (own: the uint64 division, where the scaled dividend or
+// twice the remainder passes 64 bits), it is one (one: the bisection on a
+// dividend up to 64 bits shorter than the divisor), or a remainder with bit
+// 31 set rounds down (half: 32-bit doubling, divisors of 32 bits).
+struct Quirks {
+    bool own, one, half;
+    u64 q64;
+};
+UPD_DEV Quirks quirks(const Src& a, const Src& X, const Src& B, u32 bl, bool zero, u32 S)
+{
+    const u32 bla = bits_of(a), blx = bits_of(X);
+    const bool in64 = !zero && bla + (u32)est_shift_bits((int)S) - 1u <= 64u && bl <= 64u;
+    Quirks k;
+    k.half = !in64 && bl == 32u;
+    k.one = !in64 && bl > 32u && bla != 0u && blx < bl && bl - blx <= 64u;
+    k.own = in64 && (blx > 64u || bl == 64u);
+    k.q64 = 0u;
+    if (any_lane(k.own)) {
+        Mag<2> x, y, r;
+        Mag<3> q;
+        x.w[0] = a.get(0u);
+        x.w[1] = a.get(1u);
+        y.w[0] = k.own ? B.get(0u) : 1u;
+        y.w[1] = k.own ? B.get(1u) : 0u;
+        x = mul_p10_rt<2>(x, S);
+        divmod<2, 2>(x, y, q, r);
+        const u64 b64 = ((u64)y.w[1] << 32) | y.w[0], r64 = ((u64)r.w[1] << 32) | r.w[0];
+        k.q64 = (((u64)q.w[1] << 32) | q.w[0]) + (r64 << 1 >= b64 ? 1u : 0u);
+    }
+    return k;
+}
+
+// q = round-half-up(|a| 10^S / |b|), x / 0 = |x| (ddiv's rules; faith: its
+// faithful ones); q has room for the scaled dividend, U and V as div_mem
+// says; returns the limbs
+UPD_DEV u32 div(const Dst& q, const Src& a, const Src& b, u32 S, const Dst& U, const Dst& V, bool faith)
 {
     // bit length of the lane's divisor, from the top
     u32 bl = 0, nb = 0;
@@ -526,12 +574,28 @@ UPD_DEV u32 div(const Dst& q, const Src& a, const Src& b, u32 S, const Dst& U, c
         B = V.src(nb);
         bl = zero ? 1u : bl;
     }
-    u32 rnd, n;
-    if (nb <= 4u) n = div_reg<4>(q, X.src(nx), B, bl, rnd);
-    else if (nb <= 8u) n = div_reg<8>(q, X.src(nx), B, bl, rnd);
-    else if (nb <= 16u) n = div_reg<16>(q, X.src(nx), B, bl, rnd);
-    else if (nb <= 32u) n = div_reg<32>(q, X.src(nx), B, bl, rnd);
+    Quirks k{false, false, false, 0u};
+    if (faith) k = quirks(a, X.src(nx), B, bl, zero, S);
+    u32 rnd, n, rtop = 0u;
+    if (nb <= 4u) n = div_reg<4>(q, X.src(nx), B, bl, rnd, rtop);
+    else if (nb <= 8u) n = div_reg<8>(q, X.src(nx), B, bl, rnd, rtop);
+    else if (nb <= 16u) n = div_reg<16>(q, X.src(nx), B, bl, rnd, rtop);
+    else if (nb <= 32u) n = div_reg<32>(q, X.src(nx), B, bl, rnd, rtop);
     else n = div_mem(q, U, nx, B, bl, V, rnd);
+    if (any_lane(k.own || k.one || k.half)) {
+        // a divisor of 32 bits is shifted by whole limbs: rtop is the remainder
+        if (k.half && rtop >> 31) rnd = 0u;
+        if (k.own || k.one) rnd = 0u;
+        const u32 lo = k.one ? 1u : (u32)k.q64, hi = k.one ? 0u : (u32)(k.q64 >> 32);
+        const bool put = k.own || k.one;
+        const u32 m = wave_max(put ? (hi ? 2u : lo ? 1u : 0u) : 0u);
+        const u32 n1 = m > n ? m : n;
+        for (u32 i = 0; i < n1; i++) {
+            const u32 x = i < n ? q.at(i) : 0u;
+            q.put(i, put ? (i == 0u ? lo : i == 1u ? hi : 0u) : x);
+        }
+        n = n1;
+    }
     for (u32 i = 0; any_lane(rnd != 0u); i++) {
         const u32 x = i < n ? q.at(i) : 0u;
         q.put(i, addc(x, 0u, rnd));
@@ -665,7 +729,7 @@ UPD_DEV Src eval(const Query* q, const u32* prog, const u32* cst, u32 W, u8* ws,
                 // 0 / x = +0
                 u32 any = 0;
                 for (u32 i = 0; i < a.n; i++) any |= a.at(i);
-                n = div(d, a, b, sa, U, V);
+                n = div(d, a, b, sa, U, V, q->faithful != 0u);
                 neg = any ? an ^ bn : 0u;
             }
         }
