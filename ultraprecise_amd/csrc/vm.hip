@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(64, 3)
     __shared__ i64 csum[kSumLimbs];
     const u32 lane = threadIdx.x;
     if (blockIdx.x >= h->wide_blocks) return;
-    u8* const ws = h->workspace + (usize)blockIdx.x * (usize)h->stride;
+    wide::gu8* const ws = (wide::gu8*)h->workspace + (usize)blockIdx.x * (usize)h->stride;
     u32 n = 0;
     for (int c = kFirstMultiLane; c < kNumClasses; c++) n += h->class_nitems[c];
     const u32 i0 = h->class_item0[kFirstMultiLane];
@@ -166,8 +166,8 @@ __global__ void __launch_bounds__(64, 3)
         for (u32 w0 = 0; w0 < na; w0 += kSumLimbs) {
             const u32 m = na - w0 < kSumLimbs ? na - w0 : kSumLimbs;
             for (u32 w = lane; w < m; w += 64u) {
-                const u32* a = reinterpret_cast<const u32*>(pos.b + (usize)(w0 + w) * wide::kRow);
-                const u32* b = reinterpret_cast<const u32*>(neg.b + (usize)(w0 + w) * wide::kRow);
+                const u32* a = (const u32*)(pos.b + (usize)(w0 + w) * wide::kRow);
+                const u32* b = (const u32*)(neg.b + (usize)(w0 + w) * wide::kRow);
                 i64 s = 0;
                 for (u32 k = 0; k < 64u; k += 4u) {
                     u32 x[4], y[4];

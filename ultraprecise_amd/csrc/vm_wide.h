@@ -49,15 +49,29 @@ UPD_DEV u32 wave_max(u32 x) { return x; }
 UPD_DEV u32 kword(const u32* p, u32 i) { return p[i]; }
 #endif
 
+// Workspace and columns are addressed as device memory by type: their pointers
+// come from memory, and through plain ones every access would be a flat one,
+// which may go to LDS too and end in any order, so that each wait is for all
+// that are in flight (2 M rows of the expression in vm.hip: FLAT).
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(1))) u8 gu8;
+typedef __attribute__((address_space(1))) u32 gu32;
+typedef __attribute__((address_space(1))) u32x4u gu32x4;
+#else
+typedef u8 gu8;
+typedef u32 gu32;
+typedef u32x4u gu32x4;
+#endif
+
 constexpr u32 kRow = 4u * kLanes;  // bytes of one limb of every lane
 
 // A magnitude of n limbs (n the same for all lanes): limb i of this lane is
 // the word at b + i * st + off.  In the workspace st is kRow and off the
 // lane's; a constant has st = 4 and off = 0.
 struct Src {
-    const u8* b;
+    const gu8* b;
     u32 st, off, n;
-    UPD_DEV u32 at(u32 i) const { return *reinterpret_cast<const u32*>(b + (i * st + off)); }
+    UPD_DEV u32 at(u32 i) const { return *(const gu32*)(b + (i * st + off)); }
     UPD_DEV u32 get(u32 i) const { return i < n ? at(i) : 0u; }
     // limb i of this lane, i its own (any value): zero outside
     UPD_DEV u32 sel(i32 i) const
@@ -69,10 +83,10 @@ struct Src {
 };
 
 struct Dst {
-    u8* b;
+    gu8* b;
     u32 off;
-    UPD_DEV void put(u32 i, u32 x) const { *reinterpret_cast<u32*>(b + (i * kRow + off)) = x; }
-    UPD_DEV u32 at(u32 i) const { return *reinterpret_cast<const u32*>(b + (i * kRow + off)); }
+    UPD_DEV void put(u32 i, u32 x) const { *(gu32*)(b + (i * kRow + off)) = x; }
+    UPD_DEV u32 at(u32 i) const { return *(const gu32*)(b + (i * kRow + off)); }
     UPD_DEV Src src(u32 n) const { return Src{b, kRow, off, n}; }
 };
 
@@ -607,13 +621,13 @@ UPD_DEV u32 div(const Dst& q, const Src& a, const Src& b, u32 S, const Dst& U, c
 // ---------------------------------------------------------------- columns
 
 // the compact row of B bytes into d; neg receives its sign, returns the limbs
-UPD_DEV u32 load_column(const Dst& d, const u8* col, usize row, u32 B, usize colbytes, u32& neg)
+UPD_DEV u32 load_column(const Dst& d, const gu8* col, usize row, u32 B, usize colbytes, u32& neg)
 {
     const u32 nl = (B + 3u) / 4u;
     const usize off = row * (usize)B;
     const usize d0 = off >> 2;
     const u32 sh = (u32)(off & 3u);
-    const u32* p = reinterpret_cast<const u32*>(col) + d0;
+    const gu32* p = (const gu32*)col + d0;
     const u32 tail = B & 3u ? (1u << (8u * (B & 3u))) - 1u : 0xffffffffu;
     const u32 sb = (8u * B - 1u) & 31u;
     u32 top = 0;
@@ -630,9 +644,14 @@ UPD_DEV u32 load_column(const Dst& d, const u8* col, usize row, u32 B, usize col
     if (!any_lane((d0 + ((nl + 3u) & ~3u) + 1u) * 4u > colbytes)) {
         // sixteen bytes a load, a load ahead
         u32 w[8];
-        load_dwords<4, false>(p, w);
+        auto four = [&](const gu32* at, u32* to) {
+            const u32x4u x = *(const gu32x4*)at;
+#pragma unroll
+            for (int t = 0; t < 4; t++) to[t] = x[t];
+        };
+        four(p, w);
         for (u32 g = 0; g < nl; g += 4u) {
-            if (g + 4u < nl) load_dwords<4, false>(p + g + 4u, w + 4);
+            if (g + 4u < nl) four(p + g + 4u, w + 4);
             else w[4] = p[g + 4u];
 #pragma unroll
             for (int t = 0; t < 4; t++)
@@ -661,14 +680,14 @@ struct Slots {
 };
 
 // operand word: slot or constant | constant? << 8 | shift << 16
-UPD_DEV Src operand(u32 ow, const u8* ws, const Slots* sl, const u32* cst, u32 W, u32 off, u32& neg)
+UPD_DEV Src operand(u32 ow, const gu8* ws, const Slots* sl, const u32* cst, u32 W, u32 off, u32& neg)
 {
     const u32 idx = ow & 0xffu;
     if (ow & 0x100u) {
         const u32* c = cst + idx * (W + 1u);
         const u32 h = kword(c, 0u);
         neg = h & 1u;
-        return Src{reinterpret_cast<const u8*>(c + 1), 4u, 0u, h >> 8};
+        return Src{(const gu8*)(c + 1), 4u, 0u, h >> 8};
     }
     neg = (u32)(sl->neg[idx] >> lane_id()) & 1u;
     return Src{ws + (usize)uni(sl->row[idx]) * kRow, kRow, off, uni(sl->n[idx])};
@@ -676,7 +695,7 @@ UPD_DEV Src operand(u32 ow, const u8* ws, const Slots* sl, const u32* cst, u32 W
 
 // the program for this wave's rows (`row`: the lane's); neg receives the
 // result's sign, returns the result
-UPD_DEV Src eval(const Query* q, const u32* prog, const u32* cst, u32 W, u8* ws, Slots* sl, usize row, u32& neg)
+UPD_DEV Src eval(const Query* q, const u32* prog, const u32* cst, u32 W, gu8* ws, Slots* sl, usize row, u32& neg)
 {
     const u32 off = 4u * lane_id();
     auto at = [&](u32 r) { return Dst{ws + (usize)r * kRow, off}; };
@@ -686,7 +705,7 @@ UPD_DEV Src eval(const Query* q, const u32* prog, const u32* cst, u32 W, u8* ws,
         const u32 r = kword(prog, kHeadCol + c);
         const u32 B = q->colbytes[c];
         u32 s;
-        const u32 n = load_column(at(r), q->col[c], row, B, (usize)q->rows * B, s);
+        const u32 n = load_column(at(r), (const gu8*)q->col[c], row, B, (usize)q->rows * B, s);
         sl->row[c] = r;
         sl->n[c] = n;
         sl->neg[c] = ballot(s != 0u);
