@@ -379,14 +379,17 @@ int updec_module_cache_stats(int64_t* rtc_compiles, int64_t* memory_hits, int64_
  * holds W limbs, W in {2, 4, 8, 16, 32, 64, 128, 256, 512} the smallest
  * that holds every intermediate exactly; UPDEC_EUNSUPPORTED when none does.
  * Up to 32 limbs values lie in registers; those of the 64- to 512-limb
- * classes (extended-mode programs only) in a workspace that the batch object
- * holds (at most 1 GiB, or 64 rows' worth where that is more; allocated when
- * the first such query is added and grown by later ones).
+ * classes (extended-mode programs only), and of 16- and 32-limb programs of
+ * several divisions, in a workspace that the batch object holds (at most
+ * 1 GiB, or 64 rows' worth where that is more; allocated when the first such
+ * query is added and grown by later ones; without memory for it the 16- and
+ * 32-limb programs take registers).
  *
  * A batch collects queries (program, device columns, rows, output image and
  * count) and runs them with one set of launches: persistent kernels per
  * register width take row ranges from a work counter; with use_graph the
- * launches are one HIP graph (captured at the first launch).  Results are
+ * launches of more than one kernel are one HIP graph (captured at the first
+ * such launch).  Results are
  * written to each query's 133-byte SUM image and int64 COUNT.  A batch is
  * not thread-safe across launches on different streams: use one stream per
  * batch object.  No counterpart in the reference (its queries launch one

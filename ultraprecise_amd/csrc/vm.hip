@@ -16,6 +16,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -318,9 +319,9 @@ constexpr size_t kMaxWorkspace = (size_t)1 << 30;
 constexpr size_t kWideRow = 64 * sizeof(uint32_t);   // bytes of one limb of a wave's 64 values
 
 // words of a program as the kernels read it
-uint32_t program_words(const VmProgram& p)
+uint32_t program_words(const VmProgram& p, bool wide)
 {
-    return p.wide.empty() ? 3u * (uint32_t)p.ins.size() : (uint32_t)p.wide.size();
+    return !wide ? 3u * (uint32_t)p.ins.size() : (uint32_t)p.wide.size();
 }
 
 struct Pending {
@@ -329,6 +330,7 @@ struct Pending {
     uint32_t colbytes[kMaxCols];
     int64_t rows;
     int64_t chunk;  // rows per work item of this query
+    bool wide;      // runs on the kernel of vm_wide.h
     uint8_t* image;
     int64_t* count;
 };
@@ -382,7 +384,7 @@ struct updec_batch_s {
     std::vector<Pending> pending;
     // space the pending queries take at launch
     uint32_t pend_items = 0, pend_prog_words = 0, pend_const_words = 0;
-    std::map<const VmProgram*, int> pend_programs;
+    std::set<std::pair<const VmProgram*, bool>> pend_programs;
     std::mutex mu;
 
     ~updec_batch_s()
@@ -435,16 +437,27 @@ struct updec_batch_s {
         if (want <= work_bytes) return UPDEC_OK;
         want = std::min(most, std::max(want, work_bytes + work_bytes / 2));
         // launches that use the old one are waited for
+        const size_t had = work_bytes;
         if (d_work) VMCHK(hipFree(d_work));
         d_work = nullptr;
         work_bytes = 0;
-        while (hipMalloc(reinterpret_cast<void**>(&d_work), want) != hipSuccess) {
+        auto get = [&](size_t n) {
+            if (hipMalloc(reinterpret_cast<void**>(&d_work), n) == hipSuccess) {
+                work_bytes = n;
+                return true;
+            }
             (void)hipGetLastError();
             d_work = nullptr;
+            return false;
+        };
+        while (!get(want)) {
             want /= 2;
-            if (want < 64 * stride) return api_fail(UPDEC_EHIP, "no device memory for the wide kernel's workspace");
+            if (want < 64 * stride) {
+                // the queries that are staged keep theirs
+                if (had) (void)get(had);
+                return api_fail(UPDEC_EHIP, "no device memory for the wide kernel's workspace");
+            }
         }
-        work_bytes = want;
         return UPDEC_OK;
     }
 
@@ -606,6 +619,14 @@ int updec_batch_add(updec_batch_t b, updec_vm_t v, const uint8_t* const* d_cols,
         return api_fail(UPDEC_EINVAL, "bad argument");
     std::lock_guard<std::mutex> g(b->mu);
     const VmProgram& pr = *v->prog;
+    const size_t stride = (size_t)pr.wide_rows * kWideRow;
+    bool wide = !pr.wide.empty();
+    if (wide)
+        if (int rc = b->reserve(std::max(stride, b->pend_stride))) {
+            // what the register kernels have a class for needs no workspace
+            if (pr.wclass >= kFirstMultiLane) return rc;
+            wide = false;
+        }
     // the class's tuned rows per item, raised (in steps of 64 rows) for a
     // query that would otherwise need more items than the whole batch holds
     int64_t ch = b->rows_per_item[pr.wclass];
@@ -613,13 +634,13 @@ int updec_batch_add(updec_batch_t b, updec_vm_t v, const uint8_t* const* d_cols,
     // blocks): four items per block keep the load balanced while the
     // per-item work (fetch, block reduction, partial write) stays small next
     // to the item's rows
-    const int64_t slots = 4 * (int64_t)api_device_cus() * b->blocks_per_cu[item_class(pr.wclass, !pr.wide.empty())];
+    const int64_t slots = 4 * (int64_t)api_device_cus() * b->blocks_per_cu[item_class(pr.wclass, wide)];
     const int64_t big = (rows + slots - 1) / slots;
     if (big > ch) ch = (big + 63) / 64 * 64;
     if ((rows + ch - 1) / ch > b->max_items) ch = ((rows + b->max_items - 1) / b->max_items + 63) / 64 * 64;
     const uint32_t items = (uint32_t)std::max<int64_t>(1, (rows + ch - 1) / ch);
-    const bool new_prog = b->pend_programs.find(&pr) == b->pend_programs.end();
-    const uint32_t pw = new_prog ? program_words(pr) : 0u, cw = new_prog ? (uint32_t)pr.consts.size() : 0u;
+    const bool new_prog = b->pend_programs.find({&pr, wide}) == b->pend_programs.end();
+    const uint32_t pw = new_prog ? program_words(pr, wide) : 0u, cw = new_prog ? (uint32_t)pr.consts.size() : 0u;
     if ((int)b->pending.size() >= b->max_queries || b->pend_items + items > (uint32_t)b->max_items ||
         b->pend_prog_words + pw > (uint32_t)b->max_prog_words || b->pend_const_words + cw > (uint32_t)b->max_const_words) {
         if (b->pending.empty()) return api_fail(UPDEC_EINVAL, "query does not fit an empty batch");
@@ -636,16 +657,13 @@ int updec_batch_add(updec_batch_t b, updec_vm_t v, const uint8_t* const* d_cols,
     p.chunk = ch;
     p.image = d_image;
     p.count = d_count;
-    if (!pr.wide.empty()) {
-        const size_t stride = (size_t)pr.wide_rows * kWideRow;
-        if (int rc = b->reserve(std::max(stride, b->pend_stride))) return rc;
-        b->pend_stride = std::max(stride, b->pend_stride);
-    }
+    p.wide = wide;
+    if (wide) b->pend_stride = std::max(stride, b->pend_stride);
     b->pending.push_back(p);
     b->pend_items += items;
     b->pend_prog_words += pw;
     b->pend_const_words += cw;
-    b->pend_programs[&pr] = 1;
+    b->pend_programs.insert({&pr, wide});
     if (index_out) *index_out = (int32_t)b->pending.size() - 1;
     return UPDEC_OK;
 }
@@ -680,10 +698,10 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
     // 783 -> 550.
     const int64_t spare = (b->max_items - (int64_t)b->pend_items) / (int64_t)b->pending.size();
     int64_t rows_of[kNumKernels] = {};
-    for (const Pending& p : b->pending) rows_of[std::min(item_class(p.prog->wclass, !p.prog->wide.empty()), kFirstMultiLane)] += p.rows;
+    for (const Pending& p : b->pending) rows_of[std::min(item_class(p.prog->wclass, p.wide), kFirstMultiLane)] += p.rows;
     for (Pending& p : b->pending) {
-        const int c = item_class(p.prog->wclass, !p.prog->wide.empty());
-        const int64_t T = p.prog->wide.empty() ? kBlock[c] : 64;
+        const int c = item_class(p.prog->wclass, p.wide);
+        const int64_t T = p.wide ? 64 : kBlock[c];
         const int64_t most = std::max<int64_t>(1, (p.rows + p.chunk - 1) / p.chunk) + spare;
         const int64_t even = rows_of[std::min(c, kFirstMultiLane)] / (2 * (int64_t)api_device_cus() * b->blocks_per_cu[c]);
         p.chunk = std::min(p.chunk, std::max(T, (std::max(even, (p.rows + most - 1) / most) + T - 1) / T * T));
@@ -698,7 +716,11 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
         b->clear_pending();
         return api_fail(UPDEC_EINVAL, "batch needs more work items than it was created for");
     }
-    std::map<const VmProgram*, std::pair<uint32_t, uint32_t>> placed;  // program -> (ins_off, const_off)
+    if (b->work_bytes < b->pend_stride) {
+        b->clear_pending();
+        return api_fail(UPDEC_EHIP, "the wide kernel's workspace was lost to a failed allocation");
+    }
+    std::map<std::pair<const VmProgram*, bool>, std::pair<uint32_t, uint32_t>> placed;  // program -> (ins_off, const_off)
     uint32_t prog_words = 0, const_words = 0, fill[kNumClasses];
     memcpy(fill, first, sizeof fill);
     Header& H = *b->h_hdr;
@@ -714,15 +736,15 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
     for (size_t qi = 0; qi < b->pending.size(); qi++) {
         const Pending& p = b->pending[qi];
         const VmProgram& pr = *p.prog;
-        auto it = placed.find(&pr);
+        auto it = placed.find({&pr, p.wide});
         if (it == placed.end()) {
-            const uint32_t pw = program_words(pr), cw = (uint32_t)pr.consts.size();
+            const uint32_t pw = program_words(pr, p.wide), cw = (uint32_t)pr.consts.size();
             if (prog_words + pw > (uint32_t)b->max_prog_words || const_words + cw > (uint32_t)b->max_const_words) {
                 b->clear_pending();
                 return api_fail(UPDEC_EINVAL, "batch programs exceed the staging space");
             }
-            if (!pr.wide.empty()) memcpy(b->h_prog + prog_words, pr.wide.data(), 4u * pw);
-            for (size_t k = 0; pr.wide.empty() && k < pr.ins.size(); k++) {
+            if (p.wide) memcpy(b->h_prog + prog_words, pr.wide.data(), 4u * pw);
+            for (size_t k = 0; !p.wide && k < pr.ins.size(); k++) {
                 const Ins& I = pr.ins[k];
                 uint32_t* w = b->h_prog + prog_words + 3 * k;
                 w[0] = (uint32_t)I.op | ((uint32_t)I.dst << 8) | ((uint32_t)I.arg << 16);
@@ -730,14 +752,14 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
                 w[2] = (uint32_t)I.b.kind | ((uint32_t)I.b.idx << 8) | ((uint32_t)I.b.shift << 16);
             }
             if (cw) memcpy(b->h_cst + const_words, pr.consts.data(), 4u * cw);
-            if (!pr.wide.empty())
+            if (p.wide)
                 // a constant's sign word also tells its limbs
                 for (uint32_t* k = b->h_cst + const_words; k < b->h_cst + const_words + cw; k += pr.W + 1) {
                     uint32_t n = (uint32_t)pr.W;
                     while (n > 0 && k[n] == 0u) n--;
                     *k = (*k & 1u) | (n << 8);
                 }
-            it = placed.emplace(&pr, std::make_pair(prog_words / 3u, const_words)).first;
+            it = placed.emplace(std::make_pair(&pr, p.wide), std::make_pair(prog_words / 3u, const_words)).first;
             prog_words += pw;
             const_words += cw;
         }
@@ -759,7 +781,7 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
         Q.wclass = (uint32_t)pr.wclass;
         Q.image = p.image;
         Q.count = p.count;
-        const int c = item_class(pr.wclass, !pr.wide.empty());
+        const int c = item_class(pr.wclass, p.wide);
         const int64_t ch = p.chunk;
         const uint32_t n = (uint32_t)std::max<int64_t>(1, (p.rows + ch - 1) / ch);
         Q.item0 = fill[c];
