@@ -14,9 +14,8 @@
 // stream on its own value; all group-wide decisions are uniform within a
 // group, so groups of one wave may diverge without splitting a group.
 //
-// Used by the interpreter's wide register classes (vm.hip): W = 64, 128, 256
-// and 512 limbs, where one value per lane no longer fits the register file;
-// and by the generated multi-lane calc kernels (planner.cpp, gen_calc_ml).
+// Used by the generated multi-lane calc kernels (planner.cpp, gen_calc_ml): W =
+// 64, 128, 256 and 512 limbs.
 #ifndef UPDEC_DEC_MLANE_H
 #define UPDEC_DEC_MLANE_H
 #include "dec_device.h"
@@ -627,57 +626,6 @@ UPD_DEV void store_compact_b(u8* __restrict__ out, usize row, const MDec<L>& v, 
             }
         }
     }
-}
-
-// the compact round trip of a SUM input (stored_rt): keep 8 B - 1 magnitude
-// bits, OR the bit at 8 B - 1 into the sign
-template <int L, int TPI> UPD_DEV MDec<L> stored(const MDec<L>& v, u32 B, const Grp<TPI>& g)
-{
-    MDec<L> r = v;
-    const u32 top = 8u * B - 1u;
-    u32 bit = 0;
-#pragma unroll
-    for (int i = 0; i < L; i++) {
-        const u32 lo = 32u * (g.rank * (u32)L + (u32)i);
-        if (lo > top) {
-            r.m.w[i] = 0u;
-        } else if (lo + 32u > top) {
-            const u32 k = top - lo;
-            bit = (v.m.w[i] >> k) & 1u;
-            r.m.w[i] &= k == 0u ? 0u : (0xffffffffu >> (32u - k));
-        }
-    }
-    const u64 any = g.bits(__ballot(bit ? 1 : 0));
-    r.neg |= any ? 1u : 0u;
-    return r;
-}
-
-// two's complement accumulator of W + 2 limbs: the group's W limbs plus two
-// words above them, kept (identically) on every lane of the group
-template <int L> struct Acc {
-    MMag<L> m;
-    u32 x0, x1;
-};
-
-template <int L> UPD_DEV Acc<L> acc_zero()
-{
-    Acc<L> a;
-    a.m = mzero<L>();
-    a.x0 = a.x1 = 0u;
-    return a;
-}
-
-// acc += (-1)^neg * |v|
-template <int L, int TPI> UPD_DEV void acc_add(Acc<L>& acc, const MDec<L>& v, const Grp<TPI>& g)
-{
-    MMag<L> y;
-    const u32 fm = v.neg ? 0xffffffffu : 0u;
-#pragma unroll
-    for (int i = 0; i < L; i++) y.w[i] = v.m.w[i] ^ fm;
-    const u32 c = add_mag<L, TPI>(acc.m, y, v.neg ? 1u : 0u, g);
-    const u64 s0 = (u64)acc.x0 + fm + c;
-    acc.x0 = (u32)s0;
-    acc.x1 = acc.x1 + fm + (u32)(s0 >> 32);
 }
 
 }  // namespace ml

@@ -95,7 +95,7 @@ def sin_desc(U, seed, col_id=0, P=300, S=100):
 # queries/s; rows log-uniform in [1e3, 1e7]; P from the list with S = P/3; a
 # random + - * / tree of depth 2..6 over 2..4 fresh uniform-digit columns,
 # then SUM.  Every query is served as drawn: trees whose exact
-# intermediates need more than 32 limbs run on the interpreter's multi-lane
+# intermediates need more than 32 limbs run on the interpreter's wide
 # classes (up to 512 limbs, which holds all 10,000 queries of seed 4); an
 # `accept` callback may still redraw (a test restricting the widths).
 CONFIG5 = {"queries": 10_000, "seed": 4, "rates": (200, 400, 800), "rows": (1e3, 1e7),
