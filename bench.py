@@ -474,7 +474,7 @@ def rsa(U, W, steps, cpu_rows, threads):
 def serving_bench(U, W, nq, rates, reserve_gb, jit_queries=4, saturated=True):
     """the batched serving workload: nq seeded queries at the stated
     distribution (every query as drawn: programs of up to 512 limbs run on
-    the interpreter's multi-lane classes), each on its own fresh columns
+    the interpreter's wide classes), each on its own fresh columns
     generated on the device when the query is admitted (admission by free
     device memory, hipMemGetInfo) and freed when it completes; saturated
     (all queued at once) and at Poisson arrival rates, batched (HIP graph)
