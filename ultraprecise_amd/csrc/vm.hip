@@ -111,14 +111,14 @@ __global__ void __launch_bounds__(T)
 // is one wave, an item's rows are taken 64 at a time, one lane each, with
 // every value in the block's workspace.
 //
-// What bounds it: latency of the workspace's loads (a value's limb is one
-// 256-byte line; three quarters of them hit L2) and integer issue, 40 % of the
-// time at twelve waves a CU.  The form it replaced spread every value over 16
-// to 64 lanes at the program's worst-case width.  2 M rows of
+// What bounds it: the workspace, whose lines mostly do not stay in L2 (a wave's
+// live values are some 64 KB; counters at DECIMAL(300,100): 4 TB/s read and
+// written past L2, 80 % of the wave time waiting).  The form it replaced spread
+// every value over 16 to 64 lanes at the program's worst-case width: a batch
+// of 32 queries of the serving stream, 50 M rows, 470 -> 41 ms.  1.2 M rows of
 // "((((c-c)*a)*((a/c)*(c/a)))+(b+((b/(a-a))/c)))" at DECIMAL(300,100), a
-// 256-limb program: 5.1 ms (11.6 at two waves a CU, 7.4 at four, 5.6 at
-// eight); 9 M rows 310 -> 19 ms, 2.2 M rows of a 64-limb program at
-// DECIMAL(76,25) 15.7 -> 2.0, 28,000 rows of a 128-limb one 3.4 -> 0.15.
+// 256-limb program, at two waves a CU 7.1 ms, at four 4.3, at eight 3.0, at
+// ten and twelve 2.6.
 constexpr u32 kSumLimbs = 512;   // of the accumulators at a time
 __global__ void __launch_bounds__(64, 3)
     k_vm_sum_wide(Header* h, const Query* qs, const u32* prog, const u32* cst, const Item* items, u32* partials)
