@@ -39,7 +39,7 @@ template <int TPI> struct Grp {
     UPD_DEV u64 bits(u64 ballot) const
     {
         if constexpr (TPI == 64) return ballot;
-        else return (ballot >> base) & ((1ull << TPI) - 1ull);
+        else return (word64(ballot, base) >> (base & 31u)) & (u32)((1ull << TPI) - 1ull);
     }
     // v of the group's lane src_rank (any source per lane)
     UPD_DEV u32 from(u32 v, u32 src_rank) const { return (u32)__shfl((int)v, (int)(base + src_rank), 64); }
@@ -88,7 +88,7 @@ template <int TPI> UPD_DEV u32 carry_in(const Grp<TPI>& g, bool gen, bool prop)
     const u64 G = g.bits(__ballot(gen ? 1 : 0));
     const u64 P = g.bits(__ballot(prop ? 1 : 0));
     const u64 C = (G + (G | P)) ^ P;
-    return (u32)((C >> g.rank) & 1ull);
+    return bit64(C, g.rank);
 }
 
 // a += b + c0 (c0 enters at rank 0), modulo 2^(32 W); returns the carry out

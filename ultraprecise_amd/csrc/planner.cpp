@@ -1247,6 +1247,8 @@ std::string emit_plan(Emit& E, const Plan& p, const std::vector<ColumnType>& col
         const PNode& x = p.n[i];
         std::string v = prefix + "n" + std::to_string(i);
         var[i] = v;
+        // a divisor that every lane has alike
+        const char* lit = (x.kind == PK::Div || x.kind == PK::Mod) && p.n[x.b].kind == PK::Const ? ", 1" : "";
         switch (x.kind) {
         case PK::Col: {
             int c = x.col;
@@ -1309,11 +1311,11 @@ std::string emit_plan(Emit& E, const Plan& p, const std::vector<ColumnType>& col
             break;
         case PK::Div:
             E.os << ind << "const Dec<" << x.W << "> " << v << " = ddiv<" << x.W << ", " << p.n[x.a].W << ", " << p.n[x.b].W
-                 << ", " << (p.n[x.b].S + 4) << ", " << (faith ? 1 : 0) << ">(" << var[x.a] << ", " << var[x.b] << ");\n";
+                 << ", " << (p.n[x.b].S + 4) << ", " << (faith ? 1 : 0) << lit << ">(" << var[x.a] << ", " << var[x.b] << ");\n";
             break;
         case PK::Mod:
             E.os << ind << "const Dec<" << x.W << "> " << v << " = dmod<" << x.W << ", " << p.n[x.a].W << ", " << p.n[x.b].W
-                 << ", " << (faith ? 1 : 0) << ">(" << var[x.a] << ", " << var[x.b] << ");\n";
+                 << ", " << (faith ? 1 : 0) << lit << ">(" << var[x.a] << ", " << var[x.b] << ");\n";
             break;
         case PK::Cast: {
             const PNode& A = p.n[x.a];

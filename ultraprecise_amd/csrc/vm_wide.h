@@ -340,8 +340,6 @@ UPD_DEV u32 mul(const Dst& d, const Src& x, const Src& y)
 
 // ---------------------------------------------------------------- quotient
 
-UPD_DEV u32 funnel(u32 hi, u32 lo, u32 s) { return (u32)(((((u64)hi << 32) | lo) << s) >> 32); }
-
 // quotient digit, and what it leaves of the top two words, of the three
 // words (u2, u1, u0) by (d1, d0): see divmod_digit.  r2: the third word of
 // what is left when the top words are equal and the digit saturates.
@@ -386,7 +384,7 @@ template <int NB> UPD_DEV u32 div_reg(const Dst& q, const Src& X, const Src& B, 
 #pragma unroll
         for (int i = 0; i < NB; i++) {
             const u32 hi = B.sel(i - ws);
-            V.w[i] = funnel(hi, lo, bs);
+            V.w[i] = funnel_l(hi, lo, bs);
             lo = hi;
         }
     }
@@ -399,13 +397,13 @@ template <int NB> UPD_DEV u32 div_reg(const Dst& q, const Src& X, const Src& B, 
 #pragma unroll
     for (int i = NB - 1; i >= 0; i--) {
         const u32 lo = X.sel(p + i - 1 - ws);
-        win.w[i] = funnel(hi, lo, bs);
+        win.w[i] = funnel_l(hi, lo, bs);
         hi = lo;
     }
     u32 top = 0;
     u32 next = X.sel(J - 1 - ws);
     for (i32 j = J; j >= 0; j--) {
-        const u32 u = funnel(hi, next, bs);
+        const u32 u = funnel_l(hi, next, bs);
         hi = next;
         next = X.sel(j - 2 - ws);
         const u32 u2 = win.w[NB - 1], u1 = win.w[NB - 2], u0 = win.w[NB - 3];
@@ -460,7 +458,7 @@ UPD_DEV u32 div_mem(const Dst& q, const Dst& U, u32 nx, const Src& B, u32 bl, co
         u32 hi = B.sel((i32)nb - 1 - ws);
         for (u32 i = nb; i-- > 0u;) {
             const u32 lo = B.sel((i32)i - 1 - ws);
-            V.put(i, funnel(hi, lo, bs));
+            V.put(i, funnel_l(hi, lo, bs));
             hi = lo;
         }
     }
@@ -473,7 +471,7 @@ UPD_DEV u32 div_mem(const Dst& q, const Dst& U, u32 nx, const Src& B, u32 bl, co
     u32 hi = X.sel((i32)len - 1 - ws);
     for (u32 i = len; i-- > 0u;) {
         const u32 lo = X.sel((i32)i - 1 - ws);
-        U.put(i, funnel(hi, lo, bs));
+        U.put(i, funnel_l(hi, lo, bs));
         hi = lo;
     }
     u32 top = 0;
@@ -705,7 +703,7 @@ UPD_DEV Src operand(u32 ow, const gu8* ws, const Slots* sl, const u32* cst, u32 
         neg = h & 1u;
         return Src{(const gu8*)(c + 1), 4u, 0u, h >> 8};
     }
-    neg = (u32)(sl->neg[idx] >> lane_id()) & 1u;
+    neg = bit64(sl->neg[idx], lane_id());
     return Src{ws + (usize)uni(sl->row[idx]) * kRow, kRow, off, uni(sl->n[idx])};
 }
 
