@@ -320,7 +320,8 @@ int updec_segsum_noalloc_max_segments(int precision, int32_t* max_segments);
  * and :1883-1897), i.e. Decimal(P, S, text) (src/datatypes/decimal.cu:154-165:
  * StringToDecimal :2980-3025, then cast :471-533) and ToCompactDecimal
  * (:337-341).  Row r is d_chars[d_offsets[r] .. d_offsets[r+1]) (rows + 1
- * offsets), cut at its first NUL.  The reference's character rules are kept
+ * offsets), cut at its first NUL; one whose end is not past its start is
+ * empty.  The reference's character rules are kept
  * for every byte (a non-digit c still contributes c - '0'); its reading past
  * the terminator after a trailing '.' is not: a trailing '.' ends the row.
  * The reference reports no error on this path (its overflow check is

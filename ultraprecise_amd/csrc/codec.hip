@@ -202,9 +202,10 @@ __device__ void wide_any(const char* s, u32 len, u32 frac, u32 S, u32 most, Wide
 // characters above.
 
 // The sixteen characters from s on (a byte address): the dwords that hold
-// one of them and begin before `end`, the end of the text, realigned.
-// Characters at and past `end` come out as anything.
-__device__ __forceinline__ void load_chars16(uintptr_t s, uintptr_t end, u64& x0, u64& x1)
+// one of them and begin before `end`, the last offset, realigned; or before
+// the row's own end, `left` characters on, where the offsets go down after it.
+// Characters past both come out as anything.
+__device__ __forceinline__ void load_chars16(uintptr_t s, uintptr_t end, u32 left, u64& x0, u64& x1)
 {
     const u32* p = reinterpret_cast<const u32*>(s & ~(uintptr_t)3);
     const u32 sh = (u32)(s & 3u);
@@ -212,8 +213,9 @@ __device__ __forceinline__ void load_chars16(uintptr_t s, uintptr_t end, u64& x0
     if (reinterpret_cast<uintptr_t>(p + 5) <= end) {
         load_dwords<5, false>(p, w);
     } else {
+        const uintptr_t stop = s + left > end ? s + left : end;
 #pragma unroll
-        for (int k = 0; k < 5; k++) w[k] = reinterpret_cast<uintptr_t>(p + k) < end ? p[k] : 0u;
+        for (int k = 0; k < 5; k++) w[k] = reinterpret_cast<uintptr_t>(p + k) < stop ? p[k] : 0u;
     }
     u32 t[4];
 #pragma unroll
@@ -288,7 +290,7 @@ template <int W> __device__ __forceinline__ void mul_add_word(Mag<W>& v, u32 m, 
 __device__ __forceinline__ bool plain_short(uintptr_t s, uintptr_t end, u32 len, u64& v, u32& frac, u32& neg)
 {
     u64 x0, x1;
-    load_chars16(s, end, x0, x1);
+    load_chars16(s, end, len, x0, x1);
     neg = len > 0u && (x0 & 255u) == (u64)'-' ? 1u : 0u;
     if (neg) {
         x0 = (x0 >> 8) | (x1 << 56);
@@ -308,7 +310,7 @@ template <int W> __device__ bool plain_long(uintptr_t s, uintptr_t end, u32 len,
     bool dot = false, ok = true;
     for (u32 i = 0; i < len && ok; i += 16u) {
         u64 x0, x1;
-        load_chars16(s + i, end, x0, x1);
+        load_chars16(s + i, end, len - i, x0, x1);
         const u32 cnt = len - i < 16u ? len - i : 16u;
         const Piece q = piece16(x0, x1, cnt);
         ok = ok && q.plain;
@@ -328,7 +330,7 @@ template <int W> __device__ bool plain_long(uintptr_t s, uintptr_t end, u32 len,
 __device__ __forceinline__ i64 short_any(uintptr_t s, uintptr_t end, u32 len, u32& frac, u32& neg)
 {
     u64 x0, x1;
-    load_chars16(s, end, x0, x1);
+    load_chars16(s, end, len, x0, x1);
     i64 v = 0;
     bool dot = false, force = false;
     frac = neg = 0u;
@@ -360,7 +362,7 @@ __device__ void wide_plain(uintptr_t s, uintptr_t end, u32 len, u32 frac, u32 S,
     v.n = 0u;
     for (u32 i = 0; i < len; i += 16u) {
         u64 x0, x1;
-        load_chars16(s + i, end, x0, x1);
+        load_chars16(s + i, end, len - i, x0, x1);
         const Piece q = piece16(x0, x1, len - i < 16u ? len - i : 16u);
         if (q.n > 8u) wide_mul_add(v, pow10_word(q.n - 8u), q.hi, 32u);
         wide_mul_add(v, pow10_word(q.n < 8u ? q.n : 8u), q.lo, 32u);
