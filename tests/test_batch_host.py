@@ -1,0 +1,72 @@
+"""CPU: what an interpreter batch asks of the HIP runtime, seen through a
+runtime without a device (hip_stub/fake_hip.cpp): on which device it
+allocates, what it frees and when, and what it does with little memory."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+fake.fake_log.restype = ctypes.c_char_p
+fake.fake_room.argtypes = [ctypes.c_size_t]
+fake.fake_pinned.restype = ctypes.c_void_p
+sys.path.insert(0, sys.argv[2])
+import ultraprecise_amd as U
+from ultraprecise_amd import autotune
+
+class Buf:
+    def __init__(self, ptr=4096): self.ptr = ptr
+
+def log(word=""):
+    return [l for l in fake.fake_log().decode().splitlines() if word in l]
+
+def device(d=None):
+    v = ctypes.c_int()
+    if d is not None: fake.hipSetDevice(d)
+    fake.hipGetDevice(ctypes.byref(v))
+    return v.value
+
+COLS = [(n, 38, 12) for n in "abcd"]
+C300 = [(n, 300, 100) for n in "abcd"]
+NARROW = U.VmProgram("a+b", COLS)
+# 16 limbs with three divisions: the wide kernel, or registers
+MIDDLE = U.VmProgram("a/b + c/d + b/a + " + "*".join("abc"), COLS)
+WIDE = U.VmProgram("(a+b)*c - a/d", C300)                       # 64 limbs
+WIDER = U.VmProgram("a*b*c*d*a*b*c/d", C300)
+assert (MIDDLE.width, WIDE.width) == (16, 64) and WIDER.width > 128, (MIDDLE.width, WIDE.width, WIDER.width)
+
+def add(b, prog, rows=1000):
+    return b.add(prog, [Buf() for _ in prog.cols], rows, Buf(), Buf())
+"""
+
+
+@pytest.fixture(scope="session")
+def fake(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", os.path.join(HERE, "hip_stub", "fake_hip.cpp"),
+                           "-o", out])
+
+    def run(code):
+        p = subprocess.run([sys.executable, "-c", PRELUDE + code, out, ROOT], capture_output=True, text=True, timeout=120)
+        assert p.returncode == 0, p.stdout + p.stderr
+        return p.stdout
+
+    return run
+
+
+def test_workspace_lies_on_the_batch_device(fake):
+    """queries staged by a thread whose current device is another one"""
+    fake("""
+b = U.Batch(max_queries=8, max_items=64)
+device(3)
+fake.fake_clear()
+assert add(b, WIDE) == 0 and add(b, WIDER) == 1
+assert log("hipMalloc") and all(" dev0 " in l for l in log("hipMalloc")), log()
+assert device() == 3
+""")

@@ -1,6 +1,8 @@
 // api_internal.h -- helpers shared by the C ABI translation units
 // (updec_api.hip, vm.hip, segsum.hip).
 #pragma once
+#include <hip/hip_runtime.h>
+
 #include <string>
 #include <vector>
 
@@ -8,6 +10,25 @@
 #include "planner.h"
 
 namespace updec {
+
+// the calling thread's current device is `dev` while this lives
+class OnDevice {
+  public:
+    explicit OnDevice(int dev)
+    {
+        if (hipGetDevice(&was_) != hipSuccess || was_ == dev) was_ = -1;
+        else (void)hipSetDevice(dev);
+    }
+    ~OnDevice()
+    {
+        if (was_ >= 0) (void)hipSetDevice(was_);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+
+  private:
+    int was_ = -1;
+};
 
 // record the calling thread's error message, return `code`
 int api_fail(int code, const std::string& msg);

@@ -355,6 +355,7 @@ struct updec_vm_s {
 };
 
 struct updec_batch_s {
+    int device = 0;   // the one that was current when the batch was made
     int max_queries = 0, max_items = 0, max_prog_words = 0, max_const_words = 0;
     // defaults sized so one 10^7-row query alone makes >= 4 items per CU
     int64_t rows_per_item[kNumClasses] = {8192, 8192, 4096, 2048, 1024, 512, 256, 128, 64};
@@ -435,6 +436,7 @@ struct updec_batch_s {
         const size_t most = std::max(kMaxWorkspace, 64 * stride);
         size_t want = std::min(most, (size_t)wide_grid() * stride);
         if (want <= work_bytes) return UPDEC_OK;
+        const OnDevice on(device);   // queries are staged by any thread
         want = std::min(most, std::max(want, work_bytes + work_bytes / 2));
         // launches that use the old one are waited for
         const size_t had = work_bytes;
@@ -562,6 +564,7 @@ int updec_batch_create(int32_t max_queries, int32_t max_items, updec_batch_t* ou
 {
     if (!out || max_queries <= 0 || max_items < max_queries) return api_fail(UPDEC_EINVAL, "bad argument");
     std::unique_ptr<updec_batch_s> b(new updec_batch_s());
+    VMCHK(hipGetDevice(&b->device));
     b->max_queries = max_queries;
     b->max_items = max_items;
     b->max_prog_words = max_queries * (3 * 64 + (int)wide::kHead);
