@@ -1151,9 +1151,11 @@ UPD_DEV Dec<WO> ddiv(const Dec<WA>& a, const Dec<WB>& b, u32* err = nullptr)
 #pragma unroll
         for (int i = 0; i < WX; i++) X.w[i] = bzero ? (i < WA ? a.m.w[i] : 0u) : X.w[i];
     }
+    // a dividend of up to 64 bits by a word: what the uint64 division gives
+    constexpr bool ALL_I = WB == 1 && WX <= 2;
     bool path_i = false, path_ii = false, path_iii_one = false;
     Mag<2> a2 = resize<2>(a.m), b2 = resize<2>(bs);
-    if constexpr (FAITH) {
+    if constexpr (FAITH && !ALL_I) {
         const u32 bla = bitlen(a.m), blb = bitlen(bs), blx = bitlen(X);
         path_i = !bzero && bla + (u32)est_shift_bits(S) - 1u <= 64u && blb <= 64u;
         path_ii = !path_i && blb <= 32u;
@@ -1166,7 +1168,7 @@ UPD_DEV Dec<WO> ddiv(const Dec<WA>& a, const Dec<WB>& b, u32* err = nullptr)
     // 2 R >= b, tested on the normalized remainder and divisor
     sub_to<WB>(T, vn, Rn);
     u32 rnd = ge(Rn, T) ? 1u : 0u;
-    if constexpr (FAITH) {
+    if constexpr (FAITH && !ALL_I) {
         // one-word divisor: the remainder is the top word of Rn
         if (path_ii) rnd = (u32)((Rn.w[WB - 1] >> (k & 31u)) * 2u) >= b2.w[0] ? 1u : 0u;
         if (path_iii_one) {
@@ -1179,7 +1181,15 @@ UPD_DEV Dec<WO> ddiv(const Dec<WA>& a, const Dec<WB>& b, u32* err = nullptr)
             const Mag<2> dvs = mul_p10<2, 2, S>(a2);
             Mag<3> q3;
             Mag<2> r2;
-            divmod<2, 2>(dvs, b2, q3, r2);
+            if constexpr (WB == 1) {
+                // the divisor, its shift and its reciprocal from above
+                Mag<4> un = shl_var<4>(resize<4>(dvs), k);
+                divmod_digits<2, 1, 4, 3>(un, vn, vn.w[0], 0u, recip_word(vn.w[0]), q3);
+                r2.w[0] = un.w[0] >> (k & 31u);
+                r2.w[1] = 0u;
+            } else {
+                divmod<2, 2>(dvs, b2, q3, r2);
+            }
             Mag<2> r2d;
             r2d.w[0] = r2.w[0] << 1;
             r2d.w[1] = (r2.w[1] << 1) | (r2.w[0] >> 31);
