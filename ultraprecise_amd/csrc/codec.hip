@@ -67,45 +67,17 @@ int limb_class(int B)
 
 // ---------------------------------------------------------------- ingest
 
-// scan of one row: fractional digits and sign
-struct RowScan {
-    u32 frac, neg;
-};
-
-__device__ RowScan scan_row(const char* s, u32 len)
-{
-    RowScan r{0u, 0u};
-    u32 i = 0;
-    if (len > 0 && s[0] == '-') {
-        r.neg = 1u;
-        i = 1;
-    }
-    bool dot = false;
-    for (; i < len; i++) {
-        char c = s[i];
-        if (c == 0) break;
-        if (c == '.') {
-            dot = true;
-            i++;
-            if (i >= len || s[i] == 0) break;
-            c = s[i];
-        }
-        if (dot) r.frac++;
-    }
-    return r;
-}
-
-// Rows of the long way round -- not plain (below), or cast down -- are held
-// in memory, in as many limbs as they need: rolled loops over a run-time
-// limb count keep this code's registers out of the kernel's, which the plain
-// rows need for eight waves per SIMD.
+// Rows cast down from more than 16 characters, or from any that are not plain
+// (below), are held in memory, in as many limbs as they need: rolled loops over
+// a run-time limb count keep this code's registers out of the kernel's, which
+// the plain rows need for eight waves per SIMD.
 struct WideRow {
     u32 w[32];
-    u32 n;  // limbs held; the value is modulo 2^(32 n) once n has reached `most`
+    u32 n;  // limbs held; the value is modulo 2^1024 once there are 32
 };
 
-// v = v * m + add, up to `most` limbs
-__device__ __forceinline__ void wide_mul_add(WideRow& v, u32 m, u32 add, u32 most)
+// v = v * m + add
+__device__ __forceinline__ void wide_mul_add(WideRow& v, u32 m, u32 add)
 {
     u32 c = add;
 #pragma unroll 1
@@ -114,7 +86,7 @@ __device__ __forceinline__ void wide_mul_add(WideRow& v, u32 m, u32 add, u32 mos
         v.w[i] = (u32)t;
         c = (u32)(t >> 32);
     }
-    if (c != 0u && v.n < most) v.w[v.n++] = c;
+    if (c != 0u && v.n < 32u) v.w[v.n++] = c;
 }
 
 // v = floor(v / d), d normalized to dn = d << s with reciprocal r
@@ -131,70 +103,23 @@ __device__ __forceinline__ void wide_div_word(WideRow& v, u32 dn, u32 s, u32 r)
     }
 }
 
-// to scale S: times 10^(S - frac), or floor of the division by 10^(frac - S)
-__device__ void wide_cast(WideRow& v, u32 frac, u32 S, u32 most)
+// to scale S: floor of the division by 10^(frac - S)
+__device__ void wide_cast(WideRow& v, u32 frac, u32 S)
 {
-    const bool down = frac > S;
-    u32 k = down ? frac - S : S - frac;
+    u32 k = frac - S;
     while (k != 0u) {
         const u32 step = k < 9u ? k : 9u;
         const u32 d = pow10_word(step);
-        if (down) {
-            const u32 s = (u32)__builtin_clz(d);
-            wide_div_word(v, d << s, s, recip_word(d << s));
-        } else {
-            wide_mul_add(v, d, 0u, most);
-        }
+        const u32 s = (u32)__builtin_clz(d);
+        wide_div_word(v, d << s, s, recip_word(d << s));
         k -= step;
     }
-}
-
-// StringToDecimal and the cast, modulo 2^(32 most), nine characters a fold;
-// the value is all `most` limbs of w
-__device__ void wide_any(const char* s, u32 len, u32 frac, u32 S, u32 most, WideRow& v)
-{
-    v.n = most;
-#pragma unroll 1
-    for (u32 i = 0; i < most; i++) v.w[i] = 0u;
-    auto fold = [&](u32 k, i64 chunk) {
-        const u32 m = pow10_word(k);
-        u64 c = 0;
-#pragma unroll 1
-        for (u32 i = 0; i < most; i++) {
-            const u32 a = i == 0u ? (u32)chunk : (i == 1u ? (u32)((u64)chunk >> 32) : (chunk < 0 ? 0xffffffffu : 0u));
-            const u64 t = (u64)v.w[i] * m;
-            const u64 lo = (t & 0xffffffffull) + a + (c & 0xffffffffull);
-            v.w[i] = (u32)lo;
-            c = (t >> 32) + (lo >> 32) + (c >> 32);
-        }
-    };
-    u32 i = (len > 0 && s[0] == '-') ? 1u : 0u;
-    i64 chunk = 0;
-    u32 k = 0;
-    for (; i < len; i++) {
-        char c = s[i];
-        if (c == 0) break;
-        if (c == '.') {
-            i++;
-            if (i >= len || s[i] == 0) break;
-            c = s[i];
-        }
-        chunk = chunk * 10 + ((i64)(signed char)c - '0');
-        if (++k == 9u) {
-            fold(k, chunk);
-            chunk = 0;
-            k = 0;
-        }
-    }
-    if (k) fold(k, chunk);
-    wide_cast(v, frac, S, most);
 }
 
 // ---- plain rows
 //
 // A plain row is an optional '-', then decimal digits with at most one '.'
-// among them, which is not its last character: every row that a database
-// writes.  It is parsed sixteen characters at a time in registers, without a
+// among or after them: every row that a database writes.  It is parsed sixteen characters at a time in registers, without a
 // branch per character: the dwords covering them are realigned, the '.' is
 // found and closed up, the digits are moved to the end of the sixteen bytes
 // (so that the front fills with zeros) and checked, and each four become a
@@ -224,10 +149,10 @@ __device__ __forceinline__ void load_chars16(uintptr_t s, uintptr_t end, u32 lef
     x1 = ((u64)t[3] << 32) | t[2];
 }
 
-// index of the first '.' in eight characters, 8 when there is none
-__device__ __forceinline__ u32 first_dot(u64 x)
+// index of the first C in eight characters, 8 when there is none
+template <char C> __device__ __forceinline__ u32 first_char(u64 x)
 {
-    const u64 z = x ^ 0x2e2e2e2e2e2e2e2eull;
+    const u64 z = x ^ (0x0101010101010101ull * (u64)(u8)C);
     const u64 m = (z - 0x0101010101010101ull) & ~z & 0x8080808080808080ull;
     return m ? (u32)__builtin_ctzll(m) >> 3 : 8u;
 }
@@ -246,7 +171,7 @@ struct Piece {
 __device__ __forceinline__ Piece piece16(u64 x0, u64 x1, u32 cnt)
 {
     Piece r;
-    const u32 p0 = first_dot(x0), p1 = first_dot(x1);
+    const u32 p0 = first_char<'.'>(x0), p1 = first_char<'.'>(x1);
     u32 p = p0 < 8u ? p0 : 8u + p1;
     if (p >= cnt) p = 16u;
     r.dot = p;
@@ -299,7 +224,7 @@ __device__ __forceinline__ bool plain_short(uintptr_t s, uintptr_t end, u32 len,
     const Piece q = piece16(x0, x1, len - neg);
     v = (u64)q.hi * 100000000u + q.lo;
     frac = q.dot < 16u ? len - neg - q.dot - 1u : 0u;
-    return q.plain && !(q.dot < 16u && frac == 0u);
+    return q.plain;
 }
 
 // A plain row of any length: its value modulo 2^(32 W)
@@ -322,37 +247,102 @@ template <int W> __device__ bool plain_long(uintptr_t s, uintptr_t end, u32 len,
         if (q.n > 8u) mul_add_word<W>(v, q.n == 16u ? 100000000u : pow10_word(q.n - 8u), q.hi);
         mul_add_word<W>(v, q.n >= 8u ? 100000000u : pow10_word(q.n), q.lo);
     }
-    return ok && !(dot && frac == 0u);
+    return ok;
 }
 
-// Any row of up to 16 characters by the rules above, one character a step;
-// the value fits an int64 (|v| < 208 * 10^16 / 9)
-__device__ __forceinline__ i64 short_any(uintptr_t s, uintptr_t end, u32 len, u32& frac, u32& neg)
+// Any row behind its sign by the rules above: fold(k, x) is v = v 10^k + x for
+// each sixteen characters, k of them digits, |x| < 2^59.  One character a step
+// where they are not plain, also when cut at the row's first NUL.  (Rows with a
+// NUL or a foreign character took a walk over single characters loaded one by
+// one, twice, and folds over all limbs of the output in memory: 98,000 rows of
+// DECIMAL(300,100) NUL-padded 473 -> 85 us, beginning with a space 474 -> 63;
+// 2 M of DECIMAL(15,2), one in 64 ending in a space, 222 -> 72.)
+template <class Fold> __device__ __forceinline__ void walk_any(uintptr_t s, uintptr_t end, u32 len, u32& frac, const Fold& fold)
 {
-    u64 x0, x1;
-    load_chars16(s, end, len, x0, x1);
-    i64 v = 0;
-    bool dot = false, force = false;
-    frac = neg = 0u;
+    frac = 0u;
+    bool dot = false, force = false;   // force: the character behind a '.', a digit whatever it is
 #pragma unroll 1
-    for (u32 i = 0; i < len; i++) {
-        const u32 c = (u32)x0 & 255u;
-        x0 = (x0 >> 8) | (x1 << 56);
-        x1 >>= 8;
-        if (i == 0u && c == (u32)'-') {
-            neg = 1u;
+    for (u32 i = 0; i < len; i += 16u) {
+        u64 x0, x1;
+        load_chars16(s + i, end, len - i, x0, x1);
+        u32 cnt = len - i < 16u ? len - i : 16u;
+        u32 stop = first_char<'\0'>(x0);
+        if (stop == 8u) stop += first_char<'\0'>(x1);
+        if (stop < cnt) {
+            cnt = stop;
+            len = i + stop;
+        }
+        const Piece q = piece16(x0, x1, cnt);
+        if (q.plain && !force) {
+            frac += dot ? q.n : q.dot < 16u ? cnt - q.dot - 1u : 0u;
+            dot = dot || q.dot < 16u;
+            force = q.dot < 16u && q.dot == cnt - 1u;
+            fold(q.n, (i64)((u64)q.hi * 100000000u + q.lo));
             continue;
         }
-        if (c == 0u) break;  // the row ends at its first NUL, also right after a '.'
-        if (!force && c == (u32)'.') {
-            dot = force = true;  // the next character is taken as a digit whatever it is
-            continue;
+        i64 x = 0;
+        u32 k = 0;
+#pragma unroll 1
+        for (u32 j = 0; j < cnt; j++) {
+            const u32 c = (u32)x0 & 255u;
+            x0 = (x0 >> 8) | (x1 << 56);
+            x1 >>= 8;
+            if (!force && c == (u32)'.') {
+                dot = force = true;
+                continue;
+            }
+            force = false;
+            frac += dot ? 1u : 0u;
+            x = x * 10 + ((i32)(signed char)(char)c - '0');
+            k++;
         }
-        force = false;
-        frac += dot ? 1u : 0u;
-        v = v * 10 + ((i32)(signed char)(char)c - '0');
+        fold(k, x);
     }
-    return v;
+}
+
+// to any width, modulo 2^(32 W)
+template <int W> __device__ __forceinline__ void any_row(uintptr_t s, uintptr_t end, u32 len, Mag<W>& v, u32& frac)
+{
+    v = mzero<W>();
+    walk_any(s, end, len, frac, [&](u32 k, i64 x) {
+        if (k > 8u) mul_add_word<W>(v, pow10_word(k - 8u), 0u);
+        mul_add_word<W>(v, pow10_word(k < 8u ? k : 8u), 0u);
+        const u32 ext = x < 0 ? 0xffffffffu : 0u;
+        u32 c = 0u;
+#pragma unroll
+        for (int i = 0; i < W; i++) v.w[i] = addc(v.w[i], i == 0 ? (u32)x : (i == 1 ? (u32)((u64)x >> 32) : ext), c);
+    });
+}
+
+// to be cast down: two's complement of v.n limbs, modulo 2^1024 from 32 on
+__device__ __forceinline__ void signed_mul_add(WideRow& v, u32 m, i64 add)
+{
+    const u32 ext = v.n != 0u && (i32)v.w[v.n - 1u] < 0 ? 0xffffffffu : 0u;
+    const u32 n = v.n == 0u ? 2u : v.n < 32u ? v.n + 1u : 32u;
+    u64 c = 0;
+#pragma unroll 1
+    for (u32 i = 0; i < n; i++) {
+        const u32 a = i == 0u ? (u32)add : (i == 1u ? (u32)((u64)add >> 32) : (add < 0 ? 0xffffffffu : 0u));
+        const u64 t = (u64)(i < v.n ? v.w[i] : ext) * m;
+        const u64 lo = (t & 0xffffffffull) + a + (c & 0xffffffffull);
+        v.w[i] = (u32)lo;
+        c = (t >> 32) + (lo >> 32) + (c >> 32);
+    }
+    v.n = n;
+}
+
+__device__ void wide_any(uintptr_t s, uintptr_t end, u32 len, u32 S, WideRow& v)
+{
+    v.n = 0u;
+    u32 frac;
+    walk_any(s, end, len, frac, [&](u32 k, i64 x) {
+        if (k > 8u && v.n != 0u) signed_mul_add(v, pow10_word(k - 8u), 0);
+        signed_mul_add(v, pow10_word(k < 8u ? k : 8u), x);
+    });
+    // the division is of the 1024-bit number
+    if (v.n != 0u && (i32)v.w[v.n - 1u] < 0)
+        while (v.n < 32u) v.w[v.n++] = 0xffffffffu;
+    wide_cast(v, frac, S);
 }
 
 // A plain row cast down: the division needs the whole value (modulo 2^1024,
@@ -364,10 +354,10 @@ __device__ void wide_plain(uintptr_t s, uintptr_t end, u32 len, u32 frac, u32 S,
         u64 x0, x1;
         load_chars16(s + i, end, len - i, x0, x1);
         const Piece q = piece16(x0, x1, len - i < 16u ? len - i : 16u);
-        if (q.n > 8u) wide_mul_add(v, pow10_word(q.n - 8u), q.hi, 32u);
-        wide_mul_add(v, pow10_word(q.n < 8u ? q.n : 8u), q.lo, 32u);
+        if (q.n > 8u) wide_mul_add(v, pow10_word(q.n - 8u), q.hi);
+        wide_mul_add(v, pow10_word(q.n < 8u ? q.n : 8u), q.lo);
     }
-    wide_cast(v, frac, S, 32u);
+    wide_cast(v, frac, S);
 }
 
 // rows per block of the ingest kernel, and of the two format kernels
@@ -398,14 +388,16 @@ __global__ void __launch_bounds__(kParseBlock, WO <= 16 ? 8 : 1) k_parse_compact
     if (row < rows) {
         const int64_t o0 = offsets[row], o1 = offsets[row + 1];
         const char* s = chars + o0;
-        const u32 len = o1 > o0 ? (u32)(o1 - o0) : 0u;
+        u32 len = o1 > o0 ? (u32)(o1 - o0) : 0u;
         Mag<WO> m;
         u32 neg = 0u, frac = 0u;
         bool done = false;
         const uintptr_t a = reinterpret_cast<uintptr_t>(s);
+        bool plain;
         if (len <= 16u) {
             u64 u;
-            if (plain_short(a, end, len, u, frac, neg)) {
+            plain = plain_short(a, end, len, u, frac, neg);
+            if (plain) {
                 if (S < frac) {
                     // floor(v / 10^(frac - S)), frac - S <= 15
                     u64 d = 1;
@@ -416,34 +408,26 @@ __global__ void __launch_bounds__(kParseBlock, WO <= 16 ? 8 : 1) k_parse_compact
 #pragma unroll
                 for (int i = 0; i < WO; i++) m.w[i] = i == 0 ? (u32)u : (i == 1 ? (u32)(u >> 32) : 0u);
                 done = true;
-            } else {
-                const i64 x = short_any(a, end, len, frac, neg);
-                const u32 ext = x < 0 ? 0xffffffffu : 0u;
-#pragma unroll
-                for (int i = 0; i < WO; i++) m.w[i] = i == 0 ? (u32)(u64)x : (i == 1 ? (u32)((u64)x >> 32) : ext);
-                done = S >= frac;
             }
         } else {
             neg = s[0] == '-' ? 1u : 0u;
-            const u32 n = len - neg;
-            done = plain_long<WO>(a + neg, end, n, m, frac);
-            if (done && S < frac) {
-                WideRow v;
-                wide_plain(a + neg, end, n, frac, S, v);
-#pragma unroll
-                for (int i = 0; i < WO; i++) m.w[i] = (u32)i < v.n ? v.w[i] : 0u;
-                frac = S;
-            }
+            plain = done = plain_long<WO>(a + neg, end, len - neg, m, frac);
+        }
+        if (!plain) {
+            neg = len != 0u && s[0] == '-' ? 1u : 0u;
+            any_row<WO>(a + neg, end, len - neg, m, frac);
+            done = S >= frac;
+        } else if (S < frac) {
+            done = false;
         }
         if (done) {
             if (S > frac) m = mul_p10_rt<WO>(m, S - frac);
         } else {
-            const RowScan sc = scan_row(s, len);
-            neg = sc.neg;
             WideRow v;
-            wide_any(s, len, sc.frac, S, S < sc.frac ? 32u : (u32)WO, v);
+            if (plain) wide_plain(a + neg, end, len - neg, frac, S, v);
+            else wide_any(a + neg, end, len - neg, S, v);
 #pragma unroll
-            for (int i = 0; i < WO; i++) m.w[i] = v.w[i];
+            for (int i = 0; i < WO; i++) m.w[i] = (u32)i < v.n ? v.w[i] : 0u;
         }
         // B bytes at byte offset tid * B: whole dwords (unaligned), then bytes
         u8* dst = t8 + (u32)threadIdx.x * B;
