@@ -507,7 +507,9 @@ struct FormatArgs {
 // last character back, so that every digit has its place before the length
 // is known: four at a time as a dword at the fixed distance from the end
 // that the scale gives (the '.' too).  The copy to the slots then starts
-// each row where its text starts.
+// each row where its text starts.  Divisions and digits end with the longest
+// row of the wave: with those of the column's precision, values of 3 digits in
+// DECIMAL(300,100), 200,000 rows, took 156 us instead of 51.
 //
 // What bounds it: integer issue (the divisions by 10^8 and the characters),
 // then the stores.  It had divided by 10^9, written and read every character
@@ -526,12 +528,16 @@ template <int W> __global__ void __launch_bounds__(kCodecBlock) k_format_compact
     if (row < a.rows) {
         const Dec<W> v = load_compact_rt<W>(a.col, (usize)row, a.B, (usize)a.rows * a.B);
         u32 p;  // where the text starts
+        // limbs that any row of the wave has
+        u32 most = 0;
+#pragma unroll
+        for (int i = 0; i < W; i++) most = any_lane(v.m.w[i] != 0u) ? (u32)i + 1u : most;
         if (a.hex) {
             // eight digits a limb from the top nonzero limb down, "(SSS)"
             u32 top = 0;
 #pragma unroll
             for (int i = 0; i < W; i++) {
-                if (4u * (u32)i < a.B) {
+                if ((u32)i < most) {
                     u8* d = o + a.end - 13u - 8u * (u32)i;
                     put4(d, hex4(v.m.w[i] >> 16));
                     put4(d + 4, hex4(v.m.w[i] & 0xffffu));
@@ -547,29 +553,35 @@ template <int W> __global__ void __launch_bounds__(kCodecBlock) k_format_compact
             Mag<W> x = v.m;
             const u32 point = a.S > 0u ? 1u : 0u;
             u32 n = 0;     // digits up to the highest nonzero one
-            u32 bits = 8u * a.B;
-            for (u32 j = 0; j < a.groups; j += 2u) {
+            u32 bits = 32u * most < 8u * a.B ? 32u * most : 8u * a.B;
+            // the group of four whose last is digit k
+            auto put_group = [&](u32 k, u32 c) {
+                if (k + 4u <= a.S || point == 0u) {
+                    put4(o + a.end - k - 4u, c);
+                } else if (k >= a.S) {
+                    put4(o + a.end - k - 5u, c);
+                } else {
+                    // the '.' falls inside the group
+#pragma unroll
+                    for (u32 b = 0; b < 4u; b++)
+                        o[a.end - k - 1u - b - (k + b >= a.S ? 1u : 0u)] = (u8)(c >> (8u * (3u - b)));
+                }
+            };
+            u32 j = 0;
+            for (; j < a.groups && bits != 0u; j += 2u) {
                 const u32 r = div_1e8_rem<W>(x, (bits + 31u) / 32u);
-                bits = bits > 26u ? bits - 26u : 1u;   // 10^8 > 2^26
+                bits = bits > 26u ? bits - 26u : 0u;   // 10^8 > 2^26
                 const u32 hi = r / 10000u;
 #pragma unroll
                 for (u32 h = 0; h < 2u; h++) {
                     const u32 g = h ? hi : r - 10000u * hi;
-                    const u32 k = 4u * (j + h);   // digit k is the group's last
-                    const u32 c = chars4(g);
+                    const u32 k = 4u * (j + h);
                     if (g) n = k + (g >= 1000u ? 4u : g >= 100u ? 3u : g >= 10u ? 2u : 1u);
-                    if (k + 4u <= a.S || point == 0u) {
-                        put4(o + a.end - k - 4u, c);
-                    } else if (k >= a.S) {
-                        put4(o + a.end - k - 5u, c);
-                    } else {
-                        // the '.' falls inside the group
-#pragma unroll
-                        for (u32 b = 0; b < 4u; b++)
-                            o[a.end - k - 1u - b - (k + b >= a.S ? 1u : 0u)] = (u8)(c >> (8u * (3u - b)));
-                    }
+                    put_group(k, chars4(g));
                 }
             }
+            // zeros up to the digit before the '.'
+            for (; j < a.groups && 4u * j <= a.S; j++) put_group(4u * j, 0x30303030u);
             if (point) o[a.end - 1u - a.S] = '.';
             n = n > a.S ? n : a.S + 1u;
             p = a.end - n - point - v.neg;
