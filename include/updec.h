@@ -382,9 +382,11 @@ int updec_module_cache_stats(int64_t* rtc_compiles, int64_t* memory_hits, int64_
  * Up to 32 limbs values lie in registers; those of the 64- to 512-limb
  * classes (extended-mode programs only), and of 16- and 32-limb programs of
  * several divisions, in a workspace that the batch object holds (at most
- * 1 GiB, or 64 rows' worth where that is more; allocated when the first such
- * query is added and grown by later ones; without memory for it the 16- and
- * 32-limb programs take registers).
+ * 1 GiB, or 64 blocks of 64 rows where that is more; allocated on the batch's
+ * device when the first such query is added, also while a stream is being
+ * captured, and replaced by one at least twice as large when a later one needs
+ * more, the former ones being freed with the batch; without memory for it the
+ * 16- and 32-limb programs take registers).
  *
  * A batch collects queries (program, device columns, rows, output image and
  * count) and runs them with one set of launches: persistent kernels per

@@ -70,3 +70,37 @@ assert add(b, WIDE) == 0 and add(b, WIDER) == 1
 assert log("hipMalloc") and all(" dev0 " in l for l in log("hipMalloc")), log()
 assert device() == 3
 """)
+
+
+def test_a_larger_workspace_frees_nothing(fake):
+    """hipFree waits for every stream of the device, and a captured launch may
+    still be replayed on the old workspace"""
+    fake("""
+b = U.Batch(max_queries=8, max_items=64)
+fake.fake_clear()
+for prog in (MIDDLE, WIDE, WIDER):
+    assert add(b, prog) is not None
+    b.launch(graph=False)
+got = [int(l.split()[2]) for l in log("hipMalloc")]
+assert len(got) >= 2 and all(y >= 2 * x or y == 1 << 30 for x, y in zip(got, got[1:])), log()
+assert not log("hipFree"), log()
+del b
+assert len(log("hipFree")) >= len(got)
+""")
+
+
+def test_queries_are_staged_while_a_stream_is_captured(fake):
+    """by this thread or another: the allocation is in relaxed mode, and the
+    thread's own mode is back afterwards"""
+    fake("""
+b = U.Batch(max_queries=8, max_items=64)
+fake.fake_capturing(1)
+for mode in (0, 1, 2):
+    m = ctypes.c_int(mode)
+    fake.hipThreadExchangeStreamCaptureMode(ctypes.byref(m))
+    assert add(b, (MIDDLE, WIDE, WIDER)[mode]) is not None
+    m = ctypes.c_int(0)
+    fake.hipThreadExchangeStreamCaptureMode(ctypes.byref(m))
+    assert m.value == mode
+assert len(log("hipMalloc")) >= 2
+""")

@@ -30,6 +30,24 @@ class OnDevice {
     int was_ = -1;
 };
 
+// while this lives the calling thread may allocate although a stream is being
+// captured (an allocation is no part of what a capture records)
+class AllocWhileCapturing {
+  public:
+    AllocWhileCapturing() { exchange(); }
+    ~AllocWhileCapturing() { exchange(); }
+    AllocWhileCapturing(const AllocWhileCapturing&) = delete;
+    AllocWhileCapturing& operator=(const AllocWhileCapturing&) = delete;
+
+  private:
+    void exchange()
+    {
+        if (ok_) ok_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess;
+    }
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    bool ok_ = true;
+};
+
 // record the calling thread's error message, return `code`
 int api_fail(int code, const std::string& msg);
 // compute units of the current device (cached)

@@ -365,6 +365,7 @@ struct updec_batch_s {
     // largest wide program met so far needs, at most kMaxWorkspace
     uint8_t* d_work = nullptr;
     size_t work_bytes = 0;
+    std::vector<uint8_t*> old_work;
     size_t pend_stride = 0;   // bytes per block of the pending queries' largest
     Header* h_hdr = nullptr;
     Query* h_q = nullptr;
@@ -410,6 +411,7 @@ struct updec_batch_s {
         (void)hipFree(d_cst);
         (void)hipFree(d_partials);
         (void)hipFree(d_work);
+        for (uint8_t* p : old_work) (void)hipFree(p);
     }
 
     void clear_pending()
@@ -430,36 +432,32 @@ struct updec_batch_s {
 
     // workspace for blocks of `stride` bytes: for every block of a full
     // device up to kMaxWorkspace, and where that much memory is not free, for
-    // as many as there is (64 at least)
+    // as many as there is (64 at least).  One that is too small is kept until
+    // the batch ends, not freed: launches may be running on it, which hipFree
+    // would wait for with every stream of the device, and a caller's captured
+    // launch may be replayed with it.  Each is twice as large as the last, so
+    // those kept are at most as much again.
     int reserve(size_t stride)
     {
         const size_t most = std::max(kMaxWorkspace, 64 * stride);
         size_t want = std::min(most, (size_t)wide_grid() * stride);
         if (want <= work_bytes) return UPDEC_OK;
         const OnDevice on(device);   // queries are staged by any thread
-        want = std::min(most, std::max(want, work_bytes + work_bytes / 2));
-        // launches that use the old one are waited for
-        const size_t had = work_bytes;
-        if (d_work) VMCHK(hipFree(d_work));
-        d_work = nullptr;
-        work_bytes = 0;
-        auto get = [&](size_t n) {
-            if (hipMalloc(reinterpret_cast<void**>(&d_work), n) == hipSuccess) {
-                work_bytes = n;
-                return true;
-            }
+        const AllocWhileCapturing allowed;
+        want = std::min(most, std::max(want, 2 * work_bytes));
+        uint8_t* p = nullptr;
+        while (hipMalloc(reinterpret_cast<void**>(&p), want) != hipSuccess) {
             (void)hipGetLastError();
-            d_work = nullptr;
-            return false;
-        };
-        while (!get(want)) {
+            p = nullptr;
             want /= 2;
-            if (want < 64 * stride) {
-                // the queries that are staged keep theirs
-                if (had) (void)get(had);
+            if (want < std::max(64 * stride, work_bytes + 1)) {
+                if (work_bytes >= 64 * stride) return UPDEC_OK;
                 return api_fail(UPDEC_EHIP, "no device memory for the wide kernel's workspace");
             }
         }
+        if (d_work) old_work.push_back(d_work);
+        d_work = p;
+        work_bytes = want;
         return UPDEC_OK;
     }
 
@@ -718,10 +716,6 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
     if (total > (uint32_t)b->max_items) {
         b->clear_pending();
         return api_fail(UPDEC_EINVAL, "batch needs more work items than it was created for");
-    }
-    if (b->work_bytes < b->pend_stride) {
-        b->clear_pending();
-        return api_fail(UPDEC_EHIP, "the wide kernel's workspace was lost to a failed allocation");
     }
     std::map<std::pair<const VmProgram*, bool>, std::pair<uint32_t, uint32_t>> placed;  // program -> (ins_off, const_off)
     uint32_t prog_words = 0, const_words = 0, fill[kNumClasses];
