@@ -384,9 +384,11 @@ int updec_module_cache_stats(int64_t* rtc_compiles, int64_t* memory_hits, int64_
  * several divisions, in a workspace that the batch object holds (at most
  * 1 GiB, or 64 blocks of 64 rows where that is more; allocated on the batch's
  * device when the first such query is added, also while a stream is being
- * captured, and replaced by one at least twice as large when a later one needs
- * more, the former ones being freed with the batch; without memory for it the
- * 16- and 32-limb programs take registers).
+ * captured, and replaced by a larger one when a later query needs more, the
+ * former ones being freed with the batch).  Where device memory is short it is
+ * what there is, one block at least, and asked for again when a query is added
+ * to an empty batch; with less than 64 blocks the 16- and 32-limb programs take
+ * registers.
  *
  * A batch collects queries (program, device columns, rows, output image and
  * count) and runs them with one set of launches: persistent kernels per

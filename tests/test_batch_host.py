@@ -104,3 +104,56 @@ for mode in (0, 1, 2):
     assert m.value == mode
 assert len(log("hipMalloc")) >= 2
 """)
+
+
+def test_little_memory_is_asked_for_once(fake):
+    """a workspace smaller than wanted serves the queries of one batch; the
+    next batch asks again"""
+    fake("""
+b = U.Batch(max_queries=64, max_items=1 << 12)
+fake.fake_room(100 << 20)
+for prog in (WIDE, WIDE, WIDER, WIDE):
+    assert add(b, prog) is not None
+asked = len(log("hipMalloc"))
+first = [l for l in log("hipMalloc") if l.endswith("-> 0")][-1]
+assert int(first.split()[2]) <= 100 << 20
+for prog in (WIDE, WIDER, MIDDLE) * 5:
+    assert add(b, prog) is not None
+assert len(log("hipMalloc")) == asked and not log("hipFree"), log()
+b.launch(graph=False)
+assert [l for l in log("launch") if "k_vm_sum_wide" in l]
+fake.fake_room(4 << 30)
+assert add(b, WIDER) is not None
+assert int(log("hipMalloc")[-1].split()[2]) > 500 << 20, log()
+""")
+
+
+def test_memory_for_one_block(fake):
+    """programs that have no register class run on one block; the others take
+    registers"""
+    fake("""
+b = U.Batch(max_queries=64, max_items=1 << 12)
+fake.fake_room(1 << 20)
+assert add(b, WIDE) is not None and add(b, MIDDLE) is not None
+b.launch(graph=False)
+names = " ".join(log("launch"))
+assert "k_vm_sum_wide" in names and "k_vm_sumILi16" in names, names
+assert [l for l in log("hipMalloc") if l.endswith("-> 0") and int(l.split()[2]) <= 1 << 20]
+""")
+
+
+def test_no_memory_at_all(fake):
+    fake("""
+b = U.Batch(max_queries=64, max_items=1 << 12)
+fake.fake_room(0)
+assert add(b, MIDDLE) is not None
+try:
+    add(b, WIDE)
+    raise SystemExit("accepted without a workspace")
+except U.UpdecError as e:
+    assert "workspace" in str(e)
+assert b.pending == 1 and add(b, NARROW) is not None
+b.launch(graph=False)
+names = " ".join(log("launch"))
+assert "k_vm_sum_wide" not in names and "k_vm_sumILi16" in names, names
+""")

@@ -366,6 +366,7 @@ struct updec_batch_s {
     uint8_t* d_work = nullptr;
     size_t work_bytes = 0;
     std::vector<uint8_t*> old_work;
+    bool work_short = false;  // the last allocation got less than it asked for
     size_t pend_stride = 0;   // bytes per block of the pending queries' largest
     Header* h_hdr = nullptr;
     Query* h_q = nullptr;
@@ -432,28 +433,33 @@ struct updec_batch_s {
 
     // workspace for blocks of `stride` bytes: for every block of a full
     // device up to kMaxWorkspace, and where that much memory is not free, for
-    // as many as there is (64 at least).  One that is too small is kept until
-    // the batch ends, not freed: launches may be running on it, which hipFree
-    // would wait for with every stream of the device, and a caller's captured
-    // launch may be replayed with it.  Each is twice as large as the last, so
-    // those kept are at most as much again.
+    // as many as there is.  One that is too small is kept until the batch
+    // ends, not freed: launches may be running on it, which hipFree would wait
+    // for with every stream of the device, and a caller's captured launch may
+    // be replayed with it.  Each is twice as large as the last (half as large
+    // again where memory is short), so those kept are at most as much again
+    // (twice as much).
     int reserve(size_t stride)
     {
         const size_t most = std::max(kMaxWorkspace, 64 * stride);
         size_t want = std::min(most, (size_t)wide_grid() * stride);
         if (want <= work_bytes) return UPDEC_OK;
+        const bool serves = work_bytes >= stride;
+        // what there is has to do until the next batch, which asks again
+        if (serves && work_short && !pending.empty()) return UPDEC_OK;
         const OnDevice on(device);   // queries are staged by any thread
         const AllocWhileCapturing allowed;
         want = std::min(most, std::max(want, 2 * work_bytes));
+        const size_t least = serves ? work_bytes + work_bytes / 2 : stride;
+        work_short = false;
         uint8_t* p = nullptr;
-        while (hipMalloc(reinterpret_cast<void**>(&p), want) != hipSuccess) {
+        while (want < least || hipMalloc(reinterpret_cast<void**>(&p), want) != hipSuccess) {
             (void)hipGetLastError();
             p = nullptr;
-            want /= 2;
-            if (want < std::max(64 * stride, work_bytes + 1)) {
-                if (work_bytes >= 64 * stride) return UPDEC_OK;
-                return api_fail(UPDEC_EHIP, "no device memory for the wide kernel's workspace");
-            }
+            work_short = true;
+            if (want <= least)
+                return serves ? UPDEC_OK : api_fail(UPDEC_EHIP, "no device memory for the wide kernel's workspace");
+            want = std::max(want / 2, least);
         }
         if (d_work) old_work.push_back(d_work);
         d_work = p;
@@ -622,12 +628,13 @@ int updec_batch_add(updec_batch_t b, updec_vm_t v, const uint8_t* const* d_cols,
     const VmProgram& pr = *v->prog;
     const size_t stride = (size_t)pr.wide_rows * kWideRow;
     bool wide = !pr.wide.empty();
-    if (wide)
-        if (int rc = b->reserve(std::max(stride, b->pend_stride))) {
-            // what the register kernels have a class for needs no workspace
-            if (pr.wclass >= kFirstMultiLane) return rc;
-            wide = false;
-        }
+    if (wide) {
+        const size_t block = std::max(stride, b->pend_stride);
+        const int rc = b->reserve(block);
+        // what the register kernels have a class for needs no workspace
+        if (pr.wclass < kFirstMultiLane) wide = rc == UPDEC_OK && b->work_bytes >= 64 * block;
+        else if (rc) return rc;
+    }
     // the class's tuned rows per item, raised (in steps of 64 rows) for a
     // query that would otherwise need more items than the whole batch holds
     int64_t ch = b->rows_per_item[pr.wclass];
