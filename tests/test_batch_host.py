@@ -157,3 +157,20 @@ b.launch(graph=False)
 names = " ".join(log("launch"))
 assert "k_vm_sum_wide" not in names and "k_vm_sumILi16" in names, names
 """)
+
+
+def test_kernel_time_is_read_on_the_run_device(fake):
+    """the aggregation's clock, asked for by a thread whose current device is
+    another one (the fake's kernels write no reading)"""
+    fake("""
+a = U.Agg(["a+b"], COLS)
+a.run([Buf() for _ in COLS], 1000, Buf(), Buf(), max_groups=1)
+device(2)
+fake.fake_clear()
+try:
+    a.last_kernel_ms()
+except U.UpdecError:
+    pass
+assert log() and all(" dev0" in l for l in log()), log()
+assert log("hipStreamSynchronize") and device() == 2
+""")

@@ -2106,7 +2106,10 @@ static const char* kBlockReduceCount =
 // each side of it: with them 10,007 rows ungrouped took 17.8 us instead of
 // 10.6, and 59,986,052 rows in four groups 416 instead of 402.
 static const char kClockMain[] = "  if (blockIdx.x == 0u && threadIdx.x == 0u) clk[0] = device_clock();\n";
-static const char kClockFinal[] = "  if (blockIdx.x == 0u && threadIdx.x == 0u) clk[1] = device_clock();\n";
+// It marks its reading with the run's number, and with both together, so that
+// the host knows a whole reading of the run it asks for.
+static const char kClockFinal[] =
+    "  if (blockIdx.x == 0u && threadIdx.x == 0u) { const u64 t = device_clock(); clk[1] = t; clk[2] = run; clk[3] = t ^ run; }\n";
 
 // One-pass grouped aggregation.  agg_main: each block keeps an LDS hash
 // table from the 16-bit key to a dense slot (assigned on first sight) and
@@ -2231,7 +2234,7 @@ static std::string gen_agg_onepass(const AggSpec& s, const std::vector<ColumnTyp
     for (int k = 0; k < NP; k++) navg += (s.avg_mask >> k) & 1u;
     E.os << "UPD_DEV usize rec_at(u32 i, u32 nblocks) { const u32 sl = i / nblocks; return (usize)sl * EW * nblocks + (i - sl * nblocks); }\n";
     E.os << "extern \"C\" __global__ void __launch_bounds__(" << FT << ") " << name
-         << "_final(const u32* __restrict__ rec, u32 nblocks, const u32* __restrict__ stat, u32* __restrict__ next, u32 maxg, u8* __restrict__ images, u64* __restrict__ counts, u32* __restrict__ meta, u8* __restrict__ avgs, u64* __restrict__ clk)\n{\n";
+         << "_final(const u32* __restrict__ rec, u32 nblocks, const u32* __restrict__ stat, u32* __restrict__ next, u32 maxg, u8* __restrict__ images, u64* __restrict__ counts, u32* __restrict__ meta, u8* __restrict__ avgs, u64* __restrict__ clk, u64 run)\n{\n";
     E.os << kClockFinal;
     E.os << "  const u32 tid = threadIdx.x;\n";
     E.os << "  __shared__ u32 bm[2048];\n  __shared__ u32 pre[2049];\n  __shared__ u32 part[" << FW << "];\n";
@@ -2416,7 +2419,7 @@ std::string gen_agg_kernels(const AggSpec& s, const std::vector<ColumnType>& col
 
     // final: one block per (group, plan) sum and one per group count
     E.os << "extern \"C\" __global__ void __launch_bounds__(256) " << name
-         << "_final(const u32* __restrict__ partials, u32 nblocks, u8* __restrict__ images, u64* __restrict__ counts, u64* __restrict__ clk)\n{\n";
+         << "_final(const u32* __restrict__ partials, u32 nblocks, u8* __restrict__ images, u64* __restrict__ counts, u64* __restrict__ clk, u64 run)\n{\n";
     E.os << kClockFinal;
     E.os << "  const u32 k = blockIdx.x, tid = threadIdx.x;\n";
     E.os << "  __shared__ u32 red[4 * AW2 + 8];\n";

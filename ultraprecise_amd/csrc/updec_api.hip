@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <list>
@@ -626,12 +627,30 @@ struct updec_agg_s {
     u32* h_meta = nullptr;
     u32* h_meta_dev = nullptr;  // its device address
     // clock readings of the last run, which its kernels write (start of the
-    // main kernel, start of the final one): a one-pass run's follow h_meta's
-    // keys, a two-pass run's head the allocation of the partials, which
-    // needs no pinned memory otherwise
+    // main kernel, start of the final one, the run's number, both): a one-pass
+    // run's follow h_meta's keys, a two-pass run's head the allocation of the
+    // partials, which needs no pinned memory otherwise
+    static constexpr int kClocks = 4;
     u64* d_clk = nullptr;
     const u64* clk_host = nullptr;  // where the last run's can be read; null: copy from d_clk
     bool timed = false;
+    u64 run = 0;                    // the last run's number, its own among all
+    int device = 0;                 // and where it ran
+    hipStream_t stream = nullptr;
+    hipStream_t clk_stream = nullptr;  // of the copy from d_clk
+    static u64 next_run()
+    {
+        static std::atomic<u64> last{(u64)std::chrono::steady_clock::now().time_since_epoch().count()};
+        return ++last;
+    }
+    void launched(u64 number, hipStream_t st, const u64* host)
+    {
+        run = number;
+        stream = st;
+        clk_host = host;
+        (void)hipGetDevice(&device);
+        timed = true;
+    }
     int reserve_partials(size_t words)
     {
         if (words <= partial_words) return UPDEC_OK;
@@ -650,6 +669,7 @@ struct updec_agg_s {
         if (d_bitmap) (void)hipFree(d_bitmap);
         if (d_lut) (void)hipFree(d_lut);
         if (d_clk) (void)hipFree(d_clk);
+        if (clk_stream) (void)hipStreamDestroy(clk_stream);
         if (d_meta) (void)hipFree(d_meta);
         if (h_meta) (void)hipHostFree(h_meta);
     }
@@ -1247,13 +1267,14 @@ static int agg_run_onepass(updec_agg_t a, const uint8_t* const* d_cols, const in
     const int T = a->op_block;
     const int64_t grid = agg_grid(fmain, rows, T, agg_rows_per_step(a->spec, a->types, GenOptions()));
     const size_t need = (size_t)grid * (size_t)agg_onepass_record_words(a->spec);
+    u64 run = updec_agg_s::next_run();
     if (int rc = a->reserve_partials(need)) return rc;
     if (!a->d_meta) {
         HIPCHK(hipMalloc((void**)&a->d_meta, 2 * kAggOnepassStatWords * sizeof(u32)));
         a->stat_dirty = true;
     }
     if (!a->h_meta) {
-        HIPCHK(hipHostMalloc((void**)&a->h_meta, updec_agg_s::kMetaClock * sizeof(u32) + 2 * sizeof(u64), hipHostMallocMapped | hipHostMallocCoherent));
+        HIPCHK(hipHostMalloc((void**)&a->h_meta, updec_agg_s::kMetaClock * sizeof(u32) + updec_agg_s::kClocks * sizeof(u64), hipHostMallocMapped | hipHostMallocCoherent));
         HIPCHK(hipHostGetDevicePointer((void**)&a->h_meta_dev, a->h_meta, 0));
     }
     if (a->stat_dirty) HIPCHK(hipMemsetAsync(a->d_meta, 0, 2 * kAggOnepassStatWords * sizeof(u32), st));
@@ -1273,14 +1294,13 @@ static int agg_run_onepass(updec_agg_t a, const uint8_t* const* d_cols, const in
     uint64_t* cnt = reinterpret_cast<uint64_t*>(d_counts);
     u32* meta = a->h_meta_dev;
     uint8_t* avgs = a->spec.avg_mask ? d_images + (size_t)max_groups * a->spec.plans.size() * 133 : nullptr;
-    void* pf[] = {&rec, &nb, &stat, &next, &maxg, &img, &cnt, &meta, &avgs, &clk};
+    void* pf[] = {&rec, &nb, &stat, &next, &maxg, &img, &cnt, &meta, &avgs, &clk, &run};
     const int NP = (int)a->spec.plans.size();
     HIPCHK(hipModuleLaunchKernel(ffin, (unsigned)(max_groups * (NP + 1)), 1, 1, kAggFinalThreads, 1, 1, 0, st, pf, nullptr));
     a->stat_dirty = false;
     a->stat_phase = 1 - a->stat_phase;
     HIPCHK(hipStreamSynchronize(st));
-    a->timed = true;
-    a->clk_host = reinterpret_cast<const u64*>(a->h_meta + updec_agg_s::kMetaClock);
+    a->launched(run, st, reinterpret_cast<const u64*>(a->h_meta + updec_agg_s::kMetaClock));
     if (a->h_meta[2]) {
         *overflowed = true;
         return UPDEC_OK;
@@ -1355,6 +1375,7 @@ static int agg_run_twopass(updec_agg_t a, const IterArgs* iter, const uint8_t* c
     GenOptions go;
     go.blocks = iter != nullptr;
     const int64_t grid = agg_grid(fmain, rows, T, agg_rows_per_step(a->spec, a->types, go));
+    u64 run = updec_agg_s::next_run();
     if (int rc = a->reserve_partials((size_t)grid * PW)) return rc;
     if (int krc = a->consts.upload(st)) return krc;
     AggArgs args;
@@ -1379,10 +1400,9 @@ static int agg_run_twopass(updec_agg_t a, const IterArgs* iter, const uint8_t* c
     u32 nb = (u32)grid;
     uint8_t* img = d_images;
     uint64_t* cnt = reinterpret_cast<uint64_t*>(d_counts);
-    void* pf[] = {&cp, &nb, &img, &cnt, &clk};
+    void* pf[] = {&cp, &nb, &img, &cnt, &clk, &run};
     HIPCHK(hipModuleLaunchKernel(ffin, (unsigned)(NP * ngroups + ngroups), 1, 1, 256, 1, 1, 0, st, pf, nullptr));
-    a->timed = true;
-    a->clk_host = nullptr;
+    a->launched(run, st, nullptr);
     return launch_avgs(a, d_images, d_counts, ngroups, max_groups, st);
 }
 
@@ -1444,23 +1464,34 @@ int updec_agg_run_iter(updec_agg_t a, const updec_column_iter* cols, int64_t row
 int updec_agg_last_kernel_ms(updec_agg_t a, float* ms)
 {
     if (!a || !ms || !a->timed) return fail(UPDEC_EINVAL, "no timed run");
-    u64 clk[2];
+    const OnDevice on(a->device);
+    u64 clk[updec_agg_s::kClocks];
     if (a->clk_host) {  // the run has been waited for
-        clk[0] = a->clk_host[0];
-        clk[1] = a->clk_host[1];
+        memcpy(clk, a->clk_host, sizeof(clk));
     } else {
-        HIPCHK(hipDeviceSynchronize());  // the run's stream may be a non-blocking one
-        HIPCHK(hipMemcpy(clk, a->d_clk, sizeof(clk), hipMemcpyDeviceToHost));
+        // read beside the streams: nothing is waited for but this run
+        if (!a->clk_stream) HIPCHK(hipStreamCreateWithFlags(&a->clk_stream, hipStreamNonBlocking));
+        auto read = [&]() -> int {
+            HIPCHK(hipMemcpyAsync(clk, a->d_clk, sizeof(clk), hipMemcpyDeviceToHost, a->clk_stream));
+            HIPCHK(hipStreamSynchronize(a->clk_stream));
+            return UPDEC_OK;
+        };
+        auto there = [&] { return clk[2] == a->run && clk[3] == (clk[1] ^ a->run); };
+        if (int rc = read()) return rc;
+        if (!there()) {
+            if (hipStreamSynchronize(a->stream) != hipSuccess) (void)hipGetLastError();
+            if (int rc = read()) return rc;
+        }
+        if (!there()) {  // its stream has been destroyed since
+            HIPCHK(hipDeviceSynchronize());
+            if (int rc = read()) return rc;
+        }
+        if (!there()) return fail(UPDEC_EHIP, "the last run's kernels have not run");
     }
-    static std::atomic<int> khz{0};
-    if (!khz.load()) {
-        int dev = 0, v = 0;
-        HIPCHK(hipGetDevice(&dev));
-        HIPCHK(hipDeviceGetAttribute(&v, hipDeviceAttributeWallClockRate, dev));
-        if (v <= 0) return fail(UPDEC_EHIP, "the device reports no clock rate");
-        khz.store(v);
-    }
-    *ms = (float)((double)(i64)(clk[1] - clk[0]) / khz.load());
+    int khz = 0;
+    HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, a->device));
+    if (khz <= 0) return fail(UPDEC_EHIP, "the device reports no clock rate");
+    *ms = (float)((double)(i64)(clk[1] - clk[0]) / khz);
     return UPDEC_OK;
 }
 
