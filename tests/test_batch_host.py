@@ -174,3 +174,28 @@ except U.UpdecError:
 assert log() and all(" dev0" in l for l in log()), log()
 assert log("hipStreamSynchronize") and device() == 2
 """)
+
+
+def test_items_of_wide_programs_whatever_the_register_class_is_tuned_to(fake):
+    """a 16-limb program that runs on the wide kernel takes items for its
+    waves, and as many as the batch has to spare"""
+    fake("""
+b = U.Batch(max_queries=8, max_items=1 << 16)
+
+def items(tuned, max_items_left=None):
+    if tuned: b.tune(3, tuned, 4)
+    for k in range(5):
+        assert add(b, MIDDLE, 10_000_000) is not None
+    b.launch(graph=False)
+    raw = ctypes.string_at(fake.fake_pinned(2), 24 * 65536)
+    rows = []
+    for i in range(65536):
+        r0, r1 = (int.from_bytes(raw[24 * i + o:24 * i + o + 8], "little") for o in (8, 16))
+        rows.append(r1 - r0)
+        if sum(rows) == 50_000_000: return rows
+    raise SystemExit("items do not cover the rows")
+
+assert max(items(None)) <= 2048
+assert max(items(16384)) <= 2048 and max(items(32768)) <= 2048
+assert max(items(512)) <= 1024
+""")

@@ -354,11 +354,14 @@ struct updec_vm_s {
     std::vector<uint32_t> colbytes;
 };
 
+// rows per work item unless updec_batch_tuning says otherwise, so that one
+// 10^7-row query alone makes >= 4 items per CU
+constexpr int64_t kItemRows[kNumClasses] = {8192, 8192, 4096, 2048, 1024, 512, 256, 128, 64};
+
 struct updec_batch_s {
     int device = 0;   // the one that was current when the batch was made
     int max_queries = 0, max_items = 0, max_prog_words = 0, max_const_words = 0;
-    // defaults sized so one 10^7-row query alone makes >= 4 items per CU
-    int64_t rows_per_item[kNumClasses] = {8192, 8192, 4096, 2048, 1024, 512, 256, 128, 64};
+    int64_t rows_per_item[kNumClasses];
     // (a block of the wide classes is one wave)
     int blocks_per_cu[kNumClasses] = {4, 4, 4, 4, 4, 12, 12, 12, 12};
     // workspace of the wide kernel, grown by updec_batch_add to what the
@@ -390,6 +393,7 @@ struct updec_batch_s {
     std::set<std::pair<const VmProgram*, bool>> pend_programs;
     std::mutex mu;
 
+    updec_batch_s() { std::copy(kItemRows, kItemRows + kNumClasses, rows_per_item); }
     ~updec_batch_s()
     {
         if (staged_pending && staged) (void)hipEventSynchronize(staged);
@@ -711,7 +715,12 @@ int updec_batch_launch(updec_batch_t b, int use_graph, updec_stream_t stream)
         const int c = item_class(p.prog->wclass, p.wide);
         const int64_t T = p.wide ? 64 : kBlock[c];
         const int64_t most = std::max<int64_t>(1, (p.rows + p.chunk - 1) / p.chunk) + spare;
-        const int64_t even = rows_of[std::min(c, kFirstMultiLane)] / (2 * (int64_t)api_device_cus() * b->blocks_per_cu[c]);
+        int64_t even = rows_of[std::min(c, kFirstMultiLane)] / (2 * (int64_t)api_device_cus() * b->blocks_per_cu[c]);
+        // What a register class is tuned to suits its own kernel's blocks, not
+        // the wide kernel's waves: items of 8,000 rows of 16 limbs took one of
+        // those some 10 ms, a quarter of a batch of 50 M rows.
+        if (p.wide && p.prog->wclass < kFirstMultiLane)
+            even = std::min(even, std::max(kItemRows[p.prog->wclass], p.rows / (4 * (int64_t)b->wide_grid())));
         p.chunk = std::min(p.chunk, std::max(T, (std::max(even, (p.rows + most - 1) / most) + T - 1) / T * T));
         nitems[c] += (uint32_t)std::max<int64_t>(1, (p.rows + p.chunk - 1) / p.chunk);
     }
