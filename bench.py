@@ -486,7 +486,7 @@ def serving_bench(U, W, nq, rates, reserve_gb, jit_queries=4, saturated=True):
     t0 = time.time()
     tuning = autotune.tune(U, use_cache=False)
     tune_s = time.time() - t0
-    log("serving: autotuned (rows per item, blocks per CU[, lanes]) per width class:", tuning, f"in {tune_s:.1f} s")
+    log("serving: autotuned (rows per item, blocks per CU) per width class:", tuning, f"in {tune_s:.1f} s")
     t0 = time.time()
     qs = [W.random_query(C["seed"], i) for i in range(nq)]
     progs = [U.VmProgram(q["text"], q["cols"]) for q in qs]

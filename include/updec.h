@@ -405,6 +405,9 @@ typedef struct updec_batch_s* updec_batch_t;
 int updec_vm_compile(const char* text, const updec_column_desc* cols, int ncols, int mode, updec_vm_t* out);
 int updec_vm_info(updec_vm_t v, int32_t* width, int32_t* nins, int32_t* nregs, int32_t* precision, int32_t* scale,
                   int32_t* faithful);
+/* *bytes: the workspace that a block of the batch's wide kernel takes for the
+ * program; 0 for one that runs in registers */
+int updec_vm_workspace(updec_vm_t v, int64_t* bytes);
 int updec_vm_listing(updec_vm_t v, char* buf, size_t cap, size_t* needed);
 void updec_vm_free(updec_vm_t v);
 int updec_batch_create(int32_t max_queries, int32_t max_items, updec_batch_t* out);

@@ -195,6 +195,7 @@ def _load():
         "updec_vm_compile": (ctypes.c_int, [ctypes.c_char_p, ctypes.POINTER(ColumnDesc), ctypes.c_int, ctypes.c_int,
                                             ctypes.POINTER(P)]),
         "updec_vm_info": (ctypes.c_int, [P] + [ctypes.POINTER(I32)] * 6),
+        "updec_vm_workspace": (ctypes.c_int, [P, ctypes.POINTER(I64)]),
         "updec_vm_listing": (ctypes.c_int, [P, ctypes.c_char_p, SZ, ctypes.POINTER(SZ)]),
         "updec_vm_free": (None, [P]),
         "updec_batch_create": (ctypes.c_int, [I32, I32, ctypes.POINTER(P)]),
@@ -233,7 +234,7 @@ EXPORTED = ["updec_last_error", "updec_version", "updec_init", "updec_compact_by
             "updec_agg_free", "updec_div_int64", "updec_segsum_compact", "updec_segsum_compact_noalloc",
             "updec_segsum_noalloc_max_segments", "updec_compile", "updec_launch",
             "updec_module_free", "updec_check_compile", "updec_module_cache_stats", "updec_gen_compact", "updec_gen_int32", "updec_gen_byte",
-            "updec_vm_compile", "updec_vm_info", "updec_vm_listing", "updec_vm_free", "updec_batch_create",
+            "updec_vm_compile", "updec_vm_info", "updec_vm_workspace", "updec_vm_listing", "updec_vm_free", "updec_batch_create",
             "updec_batch_tuning", "updec_batch_lanes", "updec_batch_add", "updec_batch_pending", "updec_batch_launch", "updec_batch_free",
             "updec_parse_compact", "updec_format_stride", "updec_format_compact", "updec_expr_calc_blocks",
             "updec_agg_run_blocks", "updec_expr_calc_iter", "updec_agg_run_iter", "updec_expr_source_iter",
@@ -693,7 +694,7 @@ def gen_byte_device(seed, column_id, choices, rows, row0=0, stream=None):
 
 
 VM_CLASS_WIDTHS = (2, 4, 8, 16, 32, 64, 128, 256, 512)
-VM_FIRST_MULTI_LANE = 5   # classes from here spread a value over W / 4 or W / 8 lanes
+VM_FIRST_MULTI_LANE = 5   # classes from here hold their values in a workspace
 EFULL = 5   # UPDEC_EFULL: the batch has no room for the query
 
 
@@ -713,6 +714,9 @@ class VmProgram:
         self.width, self.nins, self.nregs, self.precision, self.scale, f = [x.value for x in v]
         self.faithful = bool(f)
         self.width_class = VM_CLASS_WIDTHS.index(self.width)
+        w = ctypes.c_int64()
+        _check(_lib.updec_vm_workspace(self._h, ctypes.byref(w)))
+        self.workspace = w.value   # bytes a block of the wide kernel takes; 0: runs in registers
 
     @property
     def listing(self):

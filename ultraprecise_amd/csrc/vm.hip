@@ -553,6 +553,13 @@ int updec_vm_info(updec_vm_t v, int32_t* width, int32_t* nins, int32_t* nregs, i
     return UPDEC_OK;
 }
 
+int updec_vm_workspace(updec_vm_t v, int64_t* bytes)
+{
+    if (!v || !bytes) return api_fail(UPDEC_EINVAL, "bad argument");
+    *bytes = (int64_t)(v->prog->wide.empty() ? 0 : (size_t)v->prog->wide_rows * kWideRow);
+    return UPDEC_OK;
+}
+
 int updec_vm_listing(updec_vm_t v, char* buf, size_t cap, size_t* needed)
 {
     if (!v) return api_fail(UPDEC_EINVAL, "null program");

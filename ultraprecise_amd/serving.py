@@ -149,7 +149,7 @@ class Server:
         self.batches = [U.Batch(max_queries=self.max_batch, max_items=max_items) for _ in range(self.inflight_max)]
         for b in self.batches:
             for cls, t in (tuning or {}).items():
-                b.tune(cls, t[0], t[1], lanes=t[2] if len(t) > 2 else None)
+                b.tune(cls, t[0], t[1])
         self.programs = {}
 
     def program(self, q):
