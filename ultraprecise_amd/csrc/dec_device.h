@@ -249,7 +249,7 @@ UPD_DEV u32 after(u32 x, u32 y)
 // orders those of all rows before the first sums, so that every limb product of
 // a wide pair is held at once (14 x 14 limbs: 395 registers; 32 x 32: 6.9 KB of
 // scratch a lane).  From 8 x 8 limbs on a row waits for the one before it: a * b
-// of DECIMAL(300,100), 250,000 rows, 1243 -> 55 us; (200,66), 380,000 rows,
+// of DECIMAL(300,100), 250,000 rows, 1243 -> 58 us; (200,66), 380,000 rows,
 // 130 -> 39; (110,36), 690,000 rows, 46 -> 29.  Below that there are registers
 // enough (DECIMAL(38,12) 26 us either way).
 constexpr int kRowsInTurn = 64;
@@ -887,10 +887,8 @@ template <int W> UPD_DEV Dec<W> ddiv_rt(const Dec<W>& a, const Dec<W>& b, u32 S,
     Mag<W> X = mul_p10_rt<W>(a.m, S);
     Mag<W> bs = b.m;
     // x / 0 keeps |x|: the unscaled dividend divided by 1.  Neither operand
-    // is kept through the division (the rounding below works on the
-    // normalized remainder): at P = 300 that and the operand loads of 16
-    // bytes take the sweep expression, 1 M rows, from 688 to 454 us, with the
-    // unrolled product's rows (71-digit x*x%N*x%N, 3 M rows: 136 to 120)
+    // is kept through the division: the rounding below works on the
+    // normalized remainder
     if (any_lane(bzero)) {
         bs.w[0] |= bzero ? 1u : 0u;
 #pragma unroll
@@ -945,10 +943,6 @@ template <int W> UPD_DEV Dec<W> ddiv_rt(const Dec<W>& a, const Dec<W>& b, u32 S,
 typedef unsigned int u32x4u __attribute__((vector_size(16), aligned(4)));
 typedef unsigned int u32x2u __attribute__((vector_size(8), aligned(4)));
 
-// Decode one compact DECIMAL row (decimal.cu:168-176): B little-endian bytes
-// at row*B, sign in bit 7 of the last byte.  Loads are the aligned dwords
-// covering the row; the last rows of a column, whose covering dwords would
-// run past the column, take a byte path.
 // four, two and one dwords from a 4-byte aligned address; NT: read once
 // (streamed past the caches)
 template <bool NT> UPD_DEV u32x4u load4(const u32* p)
@@ -988,8 +982,11 @@ template <int N, bool NT = true> UPD_DEV void load_dwords(const u32* p, u32* dw)
     if constexpr ((N & 1) != 0) dw[N - 1] = load1<NT>(p + (N - 1));
 }
 
-// Decode one compact row of B bytes (B at run time) into W limbs.  The
-// caller guarantees the magnitude fits W limbs; when B > 4 W only the low
+// Decode one compact DECIMAL row (decimal.cu:168-176), B little-endian bytes at
+// row*B with the sign in bit 7 of the last byte, into W limbs, B at run time.
+// Loads are the aligned dwords covering the row; the last rows of a column,
+// whose covering dwords would run past it, are assembled from what lies inside.
+// The caller guarantees the magnitude fits W limbs; when B > 4 W only the low
 // 4 W bytes and the sign byte are read.
 template <int W, bool NT = true> UPD_DEV Dec<W> load_compact_rt(const u8* __restrict__ col, usize row, u32 B, usize colbytes)
 {
@@ -1143,9 +1140,9 @@ UPD_DEV Dec<WO> ddiv(const Dec<WA>& a, const Dec<WB>& b, u32* err = nullptr)
     Mag<WB> bs = b.m;
     // x / 0 keeps |x|: the unscaled dividend divided by 1.  Neither operand
     // is kept through the division (the rounding below works on the
-    // normalized remainder): at P = 300 that and the operand loads of 16
-    // bytes take the sweep expression, 1 M rows, from 688 to 454 us, with the
-    // unrolled product's rows (71-digit x*x%N*x%N, 3 M rows: 136 to 120)
+    // normalized remainder): that, 16-byte operand loads and unrolled product
+    // rows took (a+b)*c - a/d of DECIMAL(300,100), 1 M rows, from 688 to 454 us
+    // (now 443)
     if (any_lane(bzero)) {
         bs.w[0] |= bzero ? 1u : 0u;
 #pragma unroll

@@ -1747,33 +1747,6 @@ bool calc_one_row(const Plan& p) { return plan_out_of_line(p) && plan_ops(p) <= 
 // 1.63 ms per 10 M rows; P = 300: 16.7 -> 16.2 ms).
 int calc_block(const Plan& p) { return p.outB > 64 ? 64 : 256; }
 
-// Widest limb array a plan keeps live: a node's own limbs, and for a
-// division the window of its long division (quotient + divisor + 1 limbs).
-static int plan_peak_limbs(const Plan& p)
-{
-    int peak = 0;
-    for (const PNode& n : p.n) {
-        peak = std::max(peak, n.W);
-        if ((n.kind == PK::Div || n.kind == PK::Mod) && n.b >= 0) peak = std::max(peak, n.W + p.n[n.b].W + 1);
-    }
-    return peak;
-}
-
-// Waves per SIMD of a calc kernel, by the limbs its plan keeps live (0: the
-// compiler's choice).  64 or more take the whole register file (512 VGPRs):
-// with two waves the limb arrays spill (sweep expression, P = 300, 76 limbs,
-// 1 M rows: 507 against 776 us; P = 260, 65 limbs: 390 against 440).  48 to
-// 63 fit the half that two waves leave each, and the second wave hides the
-// first one's column loads (P = 220, 55 limbs, 1 M rows: 219 against 287 us
-// with one; P = 190, 48 limbs, 1.5 M rows: 254 against 348).  Below that the
-// compiler's choice is as fast or faster (P = 150, 2 M rows: 242 against
-// 252 us; P = 110: 133 against 159).
-static int calc_waves(const Plan& p)
-{
-    const int peak = plan_peak_limbs(p);
-    return peak >= 64 ? 1 : peak >= 48 ? 2 : 0;
-}
-
 std::string gen_calc_kernel(const Plan& p, const std::vector<ColumnType>& cols, const std::string& name, const GenOptions& o)
 {
     Emit E;
@@ -1815,11 +1788,12 @@ std::string gen_calc_kernel(const Plan& p, const std::vector<ColumnType>& cols, 
     // output (flag byte, then the compact row: GenSaveDataCode,
     // AriesExprCalcNode.cpp:76-108)
     const std::string OS = o.blocks ? "os_" : std::to_string(OB);
-    const int waves = calc_waves(p);
-    const std::string wv = std::to_string(waves);
-    const std::string waves_attr = waves ? "__attribute__((amdgpu_waves_per_eu(" + wv + ", " + wv + "))) " : "";
-    E.os << "extern \"C\" __global__ void __launch_bounds__(" << T << ") "
-         << waves_attr << name << "("
+    // Waves per SIMD are the compiler's choice.  With product rows in turn no
+    // kernel spills for it, and fewer waves only slow: DECIMAL(300,100), 500,000
+    // rows, compiler's choice / one wave / two: (a+b)*c - a/d 231 / 231 / 245 us,
+    // a / b 82 / 126 / 79, a*b + c/d 174 / 226 / 174; DECIMAL(190,63), 790,000
+    // rows: 137 / 184 / 137, 54 / 108 / 63, 132 / 179 / 133.
+    E.os << "extern \"C\" __global__ void __launch_bounds__(" << T << ") " << name << "("
          << (o.blocks ? "IterArgs" : "ColArgs") << " a)\n{\n";
     emit_const_prologue(E, {p}, one_row);
     E.os << "  __shared__ u32 tile[(" << T << " * " << (o.blocks ? OB + 1 : OB) << " + 3) / 4];\n";
