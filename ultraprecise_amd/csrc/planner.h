@@ -232,8 +232,8 @@ struct VmProgram {
     int wclass = 0, W = 0, nregs = 0, root = 0;
     int outB = 0, outP = 0, outS = 0;
     bool faithful = false;
-    // the form with its values in a workspace (vm_wide.h), for extended-mode
-    // programs of the wide classes: words, and limbs of the workspace
+    // the form with its values in a workspace (vm_wide.h), of the programs that
+    // run there (vm.h, runs_wide): words, and limbs of the workspace
     std::vector<uint32_t> wide;
     uint32_t wide_rows = 0;
     std::string text() const;       // one line per instruction

@@ -540,10 +540,8 @@ int updec_segsum_compact_noalloc(const uint8_t* d_col, int precision, int scale,
     if (rc != UPDEC_OK || ngroups == 0) return rc;
     const usize need = (usize)ngroups * (W + 2);
     if (need > kSegScratchWords)
-        return api_fail(UPDEC_EINVAL, "segments need " + std::to_string(need * 8) + " bytes of accumulators; the fixed "
-                                      "scratch holds " + std::to_string(kSegScratchWords * 8) +
-                                      " (at most " + std::to_string(kSegScratchWords / (W + 2)) +
-                                      " segments at this precision)");
+        return api_fail(UPDEC_EINVAL, "too many segments for the fixed scratch: at most " +
+                                          std::to_string(kSegScratchWords / (W + 2)) + " at this precision");
     u64* acc = nullptr;
     rc = scratch_for_current_device(&acc);
     if (rc != UPDEC_OK) return rc;
