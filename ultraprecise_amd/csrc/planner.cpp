@@ -1236,6 +1236,14 @@ static uint32_t subtree_cols(const Plan& p, int i)
 
 // Emit straight-line code for one plan; returns the variable of the root.
 // Column loads are shared across plans through `loaded`.
+// Limbs of a plan's columns up to which all of them are loaded before anything
+// is computed.  A column that is first read late in the plan has its load behind
+// a wait for the earlier ones wherever one of those is read twice: 4 M rows of
+// DECIMAL(5,1), (a+b)*c - a/d 32.0 -> 29.8 us, a*b + c*d 25.6 -> 22.8; 2.9 M of
+// DECIMAL(38,12), 70.4 -> 66.4.  Wide columns would only hold registers:
+// DECIMAL(300,100), 373,000 rows, 178 us as they are read, 203 all at once.
+constexpr int kLoadAheadLimbs = 16;
+
 std::string emit_plan(Emit& E, const Plan& p, const std::vector<ColumnType>& cols, std::vector<std::string>& loaded,
                       const std::string& ind, const std::string& prefix)
 {
@@ -1243,6 +1251,20 @@ std::string emit_plan(Emit& E, const Plan& p, const std::vector<ColumnType>& col
     const std::string nnv = prefix + "nn";
     if (E.iter) E.os << ind << "u32 " << nnv << " = 1u;\n";
     std::vector<std::string> var(p.n.size());
+    int limbs = 0;
+    std::vector<bool> seen(cols.size());
+    for (const PNode& x : p.n)
+        if (x.kind == PK::Col && !seen[x.col]) {
+            seen[x.col] = true;
+            limbs += (compact_bytes(cols[x.col].P) + 3) / 4;
+        }
+    for (const PNode& x : p.n)
+        if (!E.iter && limbs <= kLoadAheadLimbs && x.kind == PK::Col && loaded[x.col].empty()) {
+            const int B = compact_bytes(cols[x.col].P);
+            loaded[x.col] = "c" + std::to_string(x.col);
+            E.os << ind << "const Dec<" << (B + 3) / 4 << "> " << loaded[x.col] << " = col_load<" << B << ">(a, " << x.col
+                 << ", row);\n";
+        }
     for (size_t i = 0; i < p.n.size(); i++) {
         const PNode& x = p.n[i];
         std::string v = prefix + "n" + std::to_string(i);
