@@ -637,7 +637,8 @@ struct updec_agg_s {
     u64 run = 0;                    // the last run's number, its own among all
     int device = 0;                 // and where it ran
     hipStream_t stream = nullptr;
-    hipStream_t clk_stream = nullptr;  // of the copy from d_clk
+    hipStream_t clk_stream = nullptr;  // of the copy from d_clk, and where to
+    u64* h_clk = nullptr;
     static u64 next_run()
     {
         static std::atomic<u64> last{(u64)std::chrono::steady_clock::now().time_since_epoch().count()};
@@ -670,6 +671,7 @@ struct updec_agg_s {
         if (d_lut) (void)hipFree(d_lut);
         if (d_clk) (void)hipFree(d_clk);
         if (clk_stream) (void)hipStreamDestroy(clk_stream);
+        if (h_clk) (void)hipHostFree(h_clk);
         if (d_meta) (void)hipFree(d_meta);
         if (h_meta) (void)hipHostFree(h_meta);
     }
@@ -1471,17 +1473,16 @@ int updec_agg_last_kernel_ms(updec_agg_t a, float* ms)
     } else {
         // read beside the streams: nothing is waited for but this run
         if (!a->clk_stream) HIPCHK(hipStreamCreateWithFlags(&a->clk_stream, hipStreamNonBlocking));
+        if (!a->h_clk) HIPCHK(hipHostMalloc((void**)&a->h_clk, sizeof(clk), hipHostMallocDefault));
         auto read = [&]() -> int {
-            HIPCHK(hipMemcpyAsync(clk, a->d_clk, sizeof(clk), hipMemcpyDeviceToHost, a->clk_stream));
+            HIPCHK(hipMemcpyAsync(a->h_clk, a->d_clk, sizeof(clk), hipMemcpyDeviceToHost, a->clk_stream));
             HIPCHK(hipStreamSynchronize(a->clk_stream));
+            memcpy(clk, a->h_clk, sizeof(clk));
             return UPDEC_OK;
         };
         auto there = [&] { return clk[2] == a->run && clk[3] == (clk[1] ^ a->run); };
+        if (hipStreamSynchronize(a->stream) != hipSuccess) (void)hipGetLastError();
         if (int rc = read()) return rc;
-        if (!there()) {
-            if (hipStreamSynchronize(a->stream) != hipSuccess) (void)hipGetLastError();
-            if (int rc = read()) return rc;
-        }
         if (!there()) {  // its stream has been destroyed since
             HIPCHK(hipDeviceSynchronize());
             if (int rc = read()) return rc;
