@@ -248,8 +248,7 @@ int updec_agg_run(updec_agg_t a, const uint8_t* const* d_cols, const int32_t* d_
                   int32_t* ngroups_out, uint16_t* keys_out, updec_stream_t stream);
 /* device time of the last run's main aggregation kernel, in milliseconds:
  * from its start to the start of the kernel after it, by the device's clock
- * (waits for that run, while the stream that it was given exists; else for the
- * device) */
+ * (waits for that run; UPDEC_EINVAL when there is none, or it was captured) */
 int updec_agg_last_kernel_ms(updec_agg_t a, float* ms);
 /* generated source for a given group count of the two-pass form, or of the
  * one-pass form with ngroups = 0 (no device needed) */

@@ -106,6 +106,7 @@ int hipStreamCreate(void** s) { *s = malloc(1); return 0; }
 int hipStreamCreateWithFlags(void** s, unsigned) { std::lock_guard<std::mutex> g(mu); say("hipStreamCreateWithFlags"); *s = malloc(1); return 0; }
 int hipStreamDestroy(void*) { return 0; }
 int hipStreamSynchronize(void*) { std::lock_guard<std::mutex> g(mu); say("hipStreamSynchronize"); return 0; }
+int hipStreamIsCapturing(void*, int* status) { *status = capturing ? 1 : 0; return 0; }
 int hipStreamWaitEvent(void*, void*, unsigned) { return 0; }
 int hipStreamBeginCapture(void*, int) { return 0; }
 int hipStreamEndCapture(void*, void** g) { *g = malloc(1); return 0; }

@@ -172,7 +172,16 @@ try:
 except U.UpdecError:
     pass
 assert log() and all(" dev0" in l for l in log()), log()
-assert log("hipStreamSynchronize") and device() == 2
+assert log("hipDeviceSynchronize") and device() == 2
+# a captured run has no time
+fake.fake_capturing(1)
+a.run([Buf() for _ in COLS], 1000, Buf(), Buf(), max_groups=1)
+fake.fake_clear()
+try:
+    a.last_kernel_ms()
+    raise SystemExit("a captured run was timed")
+except U.UpdecError as e:
+    assert "no timed run" in str(e) and not log(), log()
 """)
 
 

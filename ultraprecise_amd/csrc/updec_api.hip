@@ -590,6 +590,45 @@ struct updec_expr_s {
     std::map<int, std::pair<ModuleP, hipFunction_t>> ml_fn;
 };
 
+// Host words that kernels write: a slot of clock readings for every aggregation
+// object, from pages of pinned memory (allocating one takes longer than a small
+// aggregation).  Slots are given back and used again; pages stay, so there are
+// as many as the objects alive at once have filled.
+class ClockSlots {
+  public:
+    static constexpr int kWords = 8;
+    static ClockSlots& get()
+    {
+        static ClockSlots* p = new ClockSlots();  // outlives every object
+        return *p;
+    }
+    hipError_t take(u64** host)
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        if (free_.empty()) {
+            u64* page = nullptr;
+            const hipError_t e = hipHostMalloc((void**)&page, kPage * sizeof(u64),
+                                               hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent);
+            if (e != hipSuccess) return e;
+            for (size_t i = 0; i < kPage; i += kWords) free_.push_back(page + i);
+        }
+        *host = free_.back();
+        free_.pop_back();
+        memset(*host, 0, kWords * sizeof(u64));
+        return hipSuccess;
+    }
+    void give(u64* host)
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        free_.push_back(host);
+    }
+
+  private:
+    static constexpr size_t kPage = 512;
+    std::mutex mu_;
+    std::vector<u64*> free_;
+};
+
 struct updec_agg_s {
     AggSpec spec;
     std::vector<ColumnType> types;
@@ -604,8 +643,6 @@ struct updec_agg_s {
     std::map<int, GenMod> by_ngroups;
     u32* d_bitmap = nullptr;
     u8* d_lut = nullptr;
-    static constexpr size_t kClockBytes = 256;
-    static constexpr size_t kMetaClock = 4 + 256;  // word of h_meta
     u32* d_partials = nullptr;
     size_t partial_words = 0;
     // one-pass grouped form
@@ -626,42 +663,51 @@ struct updec_agg_s {
     // [4..] keys
     u32* h_meta = nullptr;
     u32* h_meta_dev = nullptr;  // its device address
-    // clock readings of the last run, which its kernels write (start of the
-    // main kernel, start of the final one, the run's number, both): a one-pass
-    // run's follow h_meta's keys, a two-pass run's head the allocation of the
-    // partials, which needs no pinned memory otherwise
-    static constexpr int kClocks = 4;
-    u64* d_clk = nullptr;
-    const u64* clk_host = nullptr;  // where the last run's can be read; null: copy from d_clk
+    // clock readings of the last run, which its kernels write: start of the
+    // main kernel, start of the final one, the run's number, both
+    u64* h_clk = nullptr;
+    u64* clk_dev = nullptr;         // its device address
     bool timed = false;
     u64 run = 0;                    // the last run's number, its own among all
     int device = 0;                 // and where it ran
-    hipStream_t stream = nullptr;
-    hipStream_t clk_stream = nullptr;  // of the copy from d_clk, and where to
-    u64* h_clk = nullptr;
     static u64 next_run()
     {
         static std::atomic<u64> last{(u64)std::chrono::steady_clock::now().time_since_epoch().count()};
         return ++last;
     }
-    void launched(u64 number, hipStream_t st, const u64* host)
+    int clock_slot(u64** dev)
     {
+        if (!h_clk) {
+            HIPCHK(ClockSlots::get().take(&h_clk));
+            HIPCHK(hipHostGetDevicePointer((void**)&clk_dev, h_clk, 0));
+        }
+        *dev = clk_dev;
+        return UPDEC_OK;
+    }
+    void launched(u64 number, hipStream_t st)
+    {
+        // a captured launch has not run
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
+        timed = cs == hipStreamCaptureStatusNone;
         run = number;
-        stream = st;
-        clk_host = host;
         (void)hipGetDevice(&device);
-        timed = true;
+    }
+    bool reading(u64* start, u64* end) const
+    {
+        u64 c[4];
+        for (int i = 0; i < 4; i++) c[i] = __atomic_load_n(h_clk + i, __ATOMIC_ACQUIRE);
+        *start = c[0];
+        *end = c[1];
+        return c[2] == run && c[3] == (c[1] ^ run);
     }
     int reserve_partials(size_t words)
     {
         if (words <= partial_words) return UPDEC_OK;
-        timed = false;
-        if (d_clk) HIPCHK(hipFree(d_clk));
-        d_clk = nullptr;
+        if (d_partials) HIPCHK(hipFree(d_partials));
         d_partials = nullptr;
         partial_words = 0;
-        HIPCHK(hipMalloc((void**)&d_clk, kClockBytes + words * sizeof(u32)));
-        d_partials = reinterpret_cast<u32*>(d_clk + kClockBytes / sizeof(u64));
+        HIPCHK(hipMalloc((void**)&d_partials, words * sizeof(u32)));
         partial_words = words;
         return UPDEC_OK;
     }
@@ -669,9 +715,9 @@ struct updec_agg_s {
     {
         if (d_bitmap) (void)hipFree(d_bitmap);
         if (d_lut) (void)hipFree(d_lut);
-        if (d_clk) (void)hipFree(d_clk);
-        if (clk_stream) (void)hipStreamDestroy(clk_stream);
-        if (h_clk) (void)hipHostFree(h_clk);
+        // hipFree waits for the object's kernels, which write to the slot
+        if (d_partials) (void)hipFree(d_partials);
+        if (h_clk) ClockSlots::get().give(h_clk);
         if (d_meta) (void)hipFree(d_meta);
         if (h_meta) (void)hipHostFree(h_meta);
     }
@@ -1276,7 +1322,7 @@ static int agg_run_onepass(updec_agg_t a, const uint8_t* const* d_cols, const in
         a->stat_dirty = true;
     }
     if (!a->h_meta) {
-        HIPCHK(hipHostMalloc((void**)&a->h_meta, updec_agg_s::kMetaClock * sizeof(u32) + updec_agg_s::kClocks * sizeof(u64), hipHostMallocMapped | hipHostMallocCoherent));
+        HIPCHK(hipHostMalloc((void**)&a->h_meta, (4 + 256) * sizeof(u32), hipHostMallocMapped | hipHostMallocCoherent));
         HIPCHK(hipHostGetDevicePointer((void**)&a->h_meta_dev, a->h_meta, 0));
     }
     if (a->stat_dirty) HIPCHK(hipMemsetAsync(a->d_meta, 0, 2 * kAggOnepassStatWords * sizeof(u32), st));
@@ -1287,7 +1333,8 @@ static int agg_run_onepass(updec_agg_t a, const uint8_t* const* d_cols, const in
     AggArgs args;
     fill_args(a, &args, d_cols, d_filter, d_key0, d_key1, rows);
     u32* ovf = stat;
-    u64* clk = reinterpret_cast<u64*>(a->h_meta_dev + updec_agg_s::kMetaClock);
+    u64* clk = nullptr;
+    if (int rc = a->clock_slot(&clk)) return rc;
     void* pm[] = {&args, &ovf, &clk};
     HIPCHK(hipModuleLaunchKernel(fmain, (uint32_t)grid, 1, 1, T, 1, 1, 0, st, pm, nullptr));
     const u32* rec = a->d_partials;
@@ -1302,7 +1349,7 @@ static int agg_run_onepass(updec_agg_t a, const uint8_t* const* d_cols, const in
     a->stat_dirty = false;
     a->stat_phase = 1 - a->stat_phase;
     HIPCHK(hipStreamSynchronize(st));
-    a->launched(run, st, reinterpret_cast<const u64*>(a->h_meta + updec_agg_s::kMetaClock));
+    a->launched(run, st);
     if (a->h_meta[2]) {
         *overflowed = true;
         return UPDEC_OK;
@@ -1382,7 +1429,8 @@ static int agg_run_twopass(updec_agg_t a, const IterArgs* iter, const uint8_t* c
     if (int krc = a->consts.upload(st)) return krc;
     AggArgs args;
     IterArgs iargs;
-    u64* clk = a->d_clk;
+    u64* clk = nullptr;
+    if (int rc = a->clock_slot(&clk)) return rc;
     void* pm[2] = {nullptr, &clk};
     if (iter) {
         iargs = *iter;
@@ -1404,7 +1452,7 @@ static int agg_run_twopass(updec_agg_t a, const IterArgs* iter, const uint8_t* c
     uint64_t* cnt = reinterpret_cast<uint64_t*>(d_counts);
     void* pf[] = {&cp, &nb, &img, &cnt, &clk, &run};
     HIPCHK(hipModuleLaunchKernel(ffin, (unsigned)(NP * ngroups + ngroups), 1, 1, 256, 1, 1, 0, st, pf, nullptr));
-    a->launched(run, st, nullptr);
+    a->launched(run, st);
     return launch_avgs(a, d_images, d_counts, ngroups, max_groups, st);
 }
 
@@ -1463,36 +1511,30 @@ int updec_agg_run_iter(updec_agg_t a, const updec_column_iter* cols, int64_t row
                            ngroups_out, keys_out, S(stream));
 }
 
+// seconds that updec_agg_last_kernel_ms waits for a reading alone
+constexpr int kClockWait = 3;
+
 int updec_agg_last_kernel_ms(updec_agg_t a, float* ms)
 {
     if (!a || !ms || !a->timed) return fail(UPDEC_EINVAL, "no timed run");
-    const OnDevice on(a->device);
-    u64 clk[updec_agg_s::kClocks];
-    if (a->clk_host) {  // the run has been waited for
-        memcpy(clk, a->clk_host, sizeof(clk));
-    } else {
-        // read beside the streams: nothing is waited for but this run
-        if (!a->clk_stream) HIPCHK(hipStreamCreateWithFlags(&a->clk_stream, hipStreamNonBlocking));
-        if (!a->h_clk) HIPCHK(hipHostMalloc((void**)&a->h_clk, sizeof(clk), hipHostMallocDefault));
-        auto read = [&]() -> int {
-            HIPCHK(hipMemcpyAsync(a->h_clk, a->d_clk, sizeof(clk), hipMemcpyDeviceToHost, a->clk_stream));
-            HIPCHK(hipStreamSynchronize(a->clk_stream));
-            memcpy(clk, a->h_clk, sizeof(clk));
-            return UPDEC_OK;
-        };
-        auto there = [&] { return clk[2] == a->run && clk[3] == (clk[1] ^ a->run); };
-        if (hipStreamSynchronize(a->stream) != hipSuccess) (void)hipGetLastError();
-        if (int rc = read()) return rc;
-        if (!there()) {  // its stream has been destroyed since
+    // The reading is waited for where it is written: the run's stream may have
+    // been destroyed, and the device may have other work.  After a long time the
+    // device is waited for, so that a run which never ends there is an error.
+    u64 start = 0, end = 0;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::seconds(kClockWait);
+    for (u32 polls = 0; !a->reading(&start, &end); polls++) {
+        if (std::chrono::steady_clock::now() > until) {
+            const OnDevice on(a->device);
             HIPCHK(hipDeviceSynchronize());
-            if (int rc = read()) return rc;
+            if (!a->reading(&start, &end)) return fail(UPDEC_EHIP, "the last run's kernels have not run");
+            break;
         }
-        if (!there()) return fail(UPDEC_EHIP, "the last run's kernels have not run");
+        if (polls > 1000) std::this_thread::sleep_for(std::chrono::microseconds(20));
     }
     int khz = 0;
     HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, a->device));
     if (khz <= 0) return fail(UPDEC_EHIP, "the device reports no clock rate");
-    *ms = (float)((double)(i64)(clk[1] - clk[0]) / khz);
+    *ms = (float)((double)(i64)(end - start) / khz);
     return UPDEC_OK;
 }
 
